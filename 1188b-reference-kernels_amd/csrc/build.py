@@ -33,6 +33,7 @@ SOURCES = [
     "unpermute.hip",
     "index_select.hip",
     "grouped_gemm.hip",
+    "expert_stream.hip",
     "grouped_gemm_bwd.hip",
     "router.hip",
     "cast.hip",

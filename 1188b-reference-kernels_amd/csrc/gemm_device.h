@@ -123,6 +123,7 @@ inline int num_cus() {
 // column tile u % ntiles.
 constexpr int kTailCtr = 0;     // units handed out
 constexpr int kTailCount = 32;  // groups in the list (own 128-byte line)
+constexpr int kTailNone = 33;   // 1: another kernel has computed the whole GEMM
 constexpr int kTailList = 64;   // the groups, ascending
 #ifndef MOE_GEMM_TAILS_MIN_K
 #define MOE_GEMM_TAILS_MIN_K 4096
@@ -138,17 +139,14 @@ __device__ __forceinline__ bool has_tail(int64_t m) {
 // 256-row tiles of a group of m rows when its tail (if has_tail) is left to the list.
 __device__ __forceinline__ int main_row_tiles(int m) { return (m + 255 - kTailMaxRows) / 256; }
 
-namespace {
-
-// One workgroup of 256 threads: each thread counts the tails of its chunk of
-// groups, an exclusive scan over the threads gives the chunk's first list
-// position, then each thread lists its chunk's tail groups. Group g is rows
+// The list, by one wavefront: each lane counts the tails of its chunk of
+// groups, an exclusive scan over the lanes gives the chunk's first list
+// position, then each lane lists its chunk's tail groups. Group g is rows
 // offsets[g] .. offsets[g + 1] - 1, clamped to [0, M].
-__global__ __launch_bounds__(256) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
-  __shared__ int part[256];
-  const int t = threadIdx.x;
-  const int64_t per = (G + 255) / 256;
-  const int64_t g0 = min(G, t * per), g1 = min(G, g0 + per);
+__device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
+  const int lane = lane_id();
+  const int64_t per = (G + kWave - 1) / kWave;
+  const int64_t g0 = min(G, lane * per), g1 = min(G, g0 + per);
   auto tail_at = [&](int64_t g) {
     const int64_t lo = min(max(static_cast<int64_t>(offsets[g]), int64_t(0)), M);
     const int64_t hi = min(max(static_cast<int64_t>(offsets[g + 1]), lo), M);
@@ -156,23 +154,34 @@ __global__ __launch_bounds__(256) void tails_init_kernel(const int32_t *offsets,
   };
   int n = 0;
   for (int64_t g = g0; g < g1; ++g) n += tail_at(g) ? 1 : 0;
-  part[t] = n;
-  __syncthreads();
-  if (t == 0) {
-    int acc = 0;
-    for (int i = 0; i < 256; ++i) {
-      const int v = part[i];
-      part[i] = acc;
-      acc += v;
-    }
-    tails[kTailCount] = acc;
+  int pos = n;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int o = __shfl_up(pos, d);
+    pos += lane >= d ? o : 0;
+  }
+  if (lane == kWave - 1) {
+    tails[kTailCount] = pos;
+    tails[kTailNone] = 0;
     tails[kTailCtr] = 0;
   }
-  __syncthreads();
-  int pos = part[t];
+  pos -= n;
   for (int64_t g = g0; g < g1; ++g) {
     if (tail_at(g)) tails[kTailList + pos++] = static_cast<int>(g);
   }
+}
+
+// The list of a GEMM that needs no ping-pong kernel (one thread).
+__device__ __forceinline__ void no_tails(int *tails) {
+  tails[kTailCount] = 0;
+  tails[kTailNone] = 1;
+  tails[kTailCtr] = 0;
+}
+
+namespace {
+
+__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
+  tails_list(offsets, G, M, tails);
 }
 
 }  // namespace

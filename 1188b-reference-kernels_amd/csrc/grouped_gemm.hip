@@ -8,7 +8,8 @@
 // SwiGLU (fused, no reference function): h = silu(y[:, :F]) * y[:, F:] on the
 // fp32 accumulators, F = N / 2, rounded once to bf16.
 //
-// Three kernels: grouped_gemm_pp_kernel (last; two wavefronts per SIMD, for
+// Short groups have kernels of their own (grouped_gemm_fwd128_kernel below and
+// expert_stream.hip). For the others there are three: grouped_gemm_pp_kernel (last; two wavefronts per SIMD, for
 // K % 64 == 0 and K >= 192 with 16-byte output rows, i.e. every MoE shape, with
 // an optional 128-row form for group tails), grouped_gemm_pipe_kernel (one
 // wavefront per SIMD; the same shapes with a K tail) and grouped_gemm_kernel,
@@ -57,7 +58,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_device.h"
+#include "grouped_gemm.h"
 
 namespace moe {
 namespace {
@@ -87,36 +88,12 @@ constexpr int kGroupM = MOE_GEMM_GROUP_M;         // row tiles per tile-order gr
 #ifndef MOE_GEMM_PINGPONG
 #define MOE_GEMM_PINGPONG 1
 #endif
-constexpr int kRowBytes = kBK * 2;                // 128: one tile row in LDS
-constexpr int kChunks = kBK / 8;                  // 8 chunks of 16 bytes per row
 constexpr int kOperandBytes = 256 * kRowBytes;    // 32 KiB: one 256-row operand tile
 constexpr int kStageBytes = 2 * kOperandBytes;    // A + B
 constexpr int kStages = 2;
 constexpr int kRowsPerKiB = 1024 / kRowBytes;     // 8 rows per DMA instruction
 
-struct GemmArgs {
-  const uint16_t *a;       // A rows, or the gather source x [a_src_rows, K]
-  const int32_t *a_rows;   // gather: A row p = a[a_rows[p]] (nullptr: A row p = a[p])
-  int64_t a_src_rows;      // gather: rows of x
-  const uint16_t *w;
-  const int32_t *offsets;
-  uint16_t *out;
-  int64_t M, K, N, G;
-  int64_t ncols;   // output columns: N (NONE) or N / 2 (SWIGLU)
-  int64_t ntiles;  // column tiles per expert
-  int vec_out;     // output rows are 16-byte aligned (ncols % 8 == 0, aligned base)
-  int *tails;      // ping-pong kernel: tail list (kTail* layout) or nullptr (tails in 256-row tiles)
-  // Reduction split of the last tiles (ping-pong kernel, 0: none): the last split_tiles tiles of the
-  // static order are left to grouped_gemm_split_kernel, which computes each as split_ways ranges of
-  // split_steps K steps (the last range takes the rest) into fp32 planes of 256 x 256 (planes), and
-  // split_sum_kernel adds each tile's planes in range order and rounds once.
-  int split_tiles, split_ways, split_steps;
-  float *planes;
-};
-
 constexpr int kPpLdsBytes = 5 * 256 * 128;  // ping-pong kernel LDS: 160 KiB
-
-__device__ __forceinline__ int swz(int row) { return (row >> 1) & (kChunks - 1); }
 
 template <bool kSwiglu>
 __device__ __forceinline__ int64_t b_row_clamped(int64_t nt, int r, int64_t ncols, int64_t N) {
@@ -1384,6 +1361,12 @@ __device__ __forceinline__ void pp_body(const GemmArgs &p, char *smem, const PpT
 template <bool kSwiglu, bool kGather, bool kTails>
 __global__ __launch_bounds__(512) void grouped_gemm_pp_kernel(GemmArgs p) {
   __shared__ __attribute__((aligned(1024))) char smem[kPpLdsBytes];
+  if constexpr (kTails) {
+    if (ld_inv(p.tails, kTailNone) != 0) return;
+    // The matrix instructions of the main loop are 8 bytes long and fetched 32 at a time; four words here put the
+    // loop where it was without the test above (c5 fc1 5.30 -> 5.26 ms; 0, 8, 16 or 24 words: 5.30, 4, 20 or 28: 5.26).
+    asm volatile("s_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+  }
   pp_body<kSwiglu, kGather, 256, kTails>(p, smem, nullptr);
   if constexpr (!kTails) return;
   volatile int *bcast = reinterpret_cast<volatile int *>(smem);
@@ -1537,6 +1520,28 @@ __global__ __launch_bounds__(512) void grouped_gemm_fwd128_kernel(GemmArgs p) {
   const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
   const int m32 = static_cast<int>(p.M), g_count = static_cast<int>(p.G);
   const int ntl = static_cast<int>((N + kTN - 1) / kTN);
+  if (p.tails != nullptr) {
+    // Only if every group fits one row tile; otherwise the ping-pong kernel that follows takes them all, and
+    // needs its list.
+    bool longer = false;
+    for (int g = threadIdx.x; g < g_count; g += 512) {
+      const int lo = min(max(p.offsets[g], 0), m32);
+      longer |= min(max(p.offsets[g + 1], lo), m32) - lo > kTM;
+    }
+    volatile int *any = reinterpret_cast<volatile int *>(smem);
+    const bool wave_any = __ballot(longer) != 0;
+    if (lane == 0) any[wave] = wave_any;
+    __syncthreads();
+    int found = 0;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) found |= any[w];
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(found)) {
+      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails);
+      return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) no_tails(p.tails);
+  }
 
   // ---- tile walker (every wavefront walks the same tiles): group by group, row tile-major
   struct Tile {
@@ -1727,6 +1732,16 @@ bool tails_apply(int64_t M_total, int64_t K, int64_t G) {
   return K % moe::gemm::kBK == 0 && (K >= moe::gemm::kTailsMinK || M_total < 256 * G);
 }
 
+// Mean rows per group up to which the weights are streamed (expert_stream.hip). With even groups of 16, 24, 32 rows
+// the stream takes 541, 546, 552 us against the ping-pong kernel's 626-629 (64 groups, K 7168, N 4096, SwiGLU, gather)
+// and, plain, 259 and 282 us at 16 and 30 rows against the 128-row tiles' 267 and 286 (40 groups, K 2560, N 8192;
+// 1.5% slower at K 8192, N 5120, where 160-column tiles make whole rounds). Skewed routing (the largest group five
+// times the mean) at 32 rows on average: 465 and 475 us, at 64 it is 10% slower.
+#ifndef MOE_STREAM_ROWS
+#define MOE_STREAM_ROWS 32
+#endif
+constexpr int64_t kStreamRows = MOE_STREAM_ROWS;
+
 // Reduction split plan of a one-group GEMM whose 256-row tiles leave the last
 // round at most half full (e.g. 320 tiles on 256 CUs): the last `tiles` tiles
 // run as `ways` K ranges each, one unit per CU, after the other tiles.
@@ -1822,27 +1837,49 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
   const bool pipe = K > 2 * kBK && p.vec_out && ncols < (int64_t(1) << 22) && (!gather || M_total < (int64_t(1) << 29));
   // The ping-pong kernel: the same conditions, whole K steps and row numbers in 31 bits.
   const bool pingpong = MOE_GEMM_PINGPONG && pipe && K % kBK == 0 && M_total < (int64_t(1) << 31);
-  // Groups of at most 128 rows on average, plain epilogue, A rows in place: 128-row tiles with their own
-  // loading wavefronts (no workspace).
-  if (MOE_GEMM_FWD128 && pingpong && !swiglu && !gather && M_total <= 128 * G) {
-    const int64_t P = std::max<int64_t>(8, num_cus() / 8 * 8);
-    switch (MOE_GEMM_FWD128_NB ? MOE_GEMM_FWD128_NB : fwd128_nb(M_total, N, G, P)) {
-      case 4: grouped_gemm_fwd128_kernel<4><<<dim3(P), dim3(512), 0, s>>>(p); break;
-      case 5: grouped_gemm_fwd128_kernel<5><<<dim3(P), dim3(512), 0, s>>>(p); break;
-      default: grouped_gemm_fwd128_kernel<6><<<dim3(P), dim3(512), 0, s>>>(p); break;
-    }
+  p.tails = nullptr;
+  p.split_tiles = p.split_ways = p.split_steps = 0;
+  p.planes = nullptr;
+  // A few rows per group: the stream of the weights.
+  if (pingpong && M_total <= kStreamRows * G && ncols < (int64_t(1) << 19)) {
+    launch_expert_stream(p, swiglu, gather, s);
     return check_launch(fn);
+  }
+  const bool tail_ws = pingpong && tails_apply(M_total, K, G) && workspace != nullptr && workspace_bytes >= tails_bytes(G) &&
+                       is_aligned(workspace, 256);
+  // Groups of at most 128 rows on average: the kernels for short groups, where the groups are short. With a workspace
+  // they look at the groups first and leave a skewed split, in which a few groups hold most of the rows, to the
+  // ping-pong kernel, whose tail list the first launch then makes (a few us for the launch that finds nothing to do).
+  // Plain, 1023 tokens over 64 experts top-8 (K 2048, N 7168): 588 us in 128-row tiles throughout, 426 us this way;
+  // 40 even groups of 102 rows (K 8192, N 5120): 664 us in 128-row tiles, 735 in the ping-pong kernel's. SwiGLU and
+  // gather, 64 even groups of 48 and 64 rows (K 7168, N 4096): 633 and 636 us in the ping-pong kernel's tail tiles,
+  // 574 and 603 streamed; of 100 rows 649 against 691.
+  bool list_made = false;
+  if (pingpong && M_total <= 128 * G) {
+    const bool look = tail_ws && M_total > 128;  // (otherwise no group has more)
+    if (look) p.tails = static_cast<int *>(workspace);
+    if (MOE_GEMM_FWD128 && !swiglu && !gather) {
+      // Plain epilogue, A rows in place: 128-row tiles with their own loading wavefronts.
+      const int64_t P = std::max<int64_t>(8, num_cus() / 8 * 8);
+      switch (MOE_GEMM_FWD128_NB ? MOE_GEMM_FWD128_NB : fwd128_nb(M_total, N, G, P)) {
+        case 4: grouped_gemm_fwd128_kernel<4><<<dim3(P), dim3(512), 0, s>>>(p); break;
+        case 5: grouped_gemm_fwd128_kernel<5><<<dim3(P), dim3(512), 0, s>>>(p); break;
+        default: grouped_gemm_fwd128_kernel<6><<<dim3(P), dim3(512), 0, s>>>(p); break;
+      }
+      if (!look) return check_launch(fn);
+      list_made = true;
+    } else if (look && M_total <= 64 * G && ncols < (int64_t(1) << 19)) {
+      launch_expert_stream(p, swiglu, gather, s);
+      list_made = true;
+    }
   }
   // With a workspace and a long reduction, group tails of at most 128 rows
   // are listed first and computed as 128-row tiles after the 256-row ones
   // (with short reductions the 128-row tiles' start and drain measured slower
   // than the padding rows they save).
-  p.tails = nullptr;
-  p.split_tiles = p.split_ways = p.split_steps = 0;
-  p.planes = nullptr;
   // One group whose last round of tiles is sparse: with a large enough workspace, a reduction split of
   // those tiles (the results differ from the unsplit ones only in the order of their fp32 partial sums).
-  const SplitPlan sp = pingpong ? split_plan(M_total, K, N, G, num_cus()) : SplitPlan{};
+  const SplitPlan sp = pingpong && !list_made ? split_plan(M_total, K, N, G, num_cus()) : SplitPlan{};
   if (sp.tiles > 0 && workspace != nullptr && workspace_bytes >= sp.bytes && is_aligned(workspace, 256)) {
     p.split_tiles = sp.tiles;
     p.split_ways = sp.ways;
@@ -1872,10 +1909,9 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
     }
     return check_launch(fn);
   }
-  if (pingpong && tails_apply(M_total, K, G) && workspace != nullptr && workspace_bytes >= tails_bytes(G) &&
-      is_aligned(workspace, 256)) {
+  if (tail_ws) {
     p.tails = static_cast<int *>(workspace);
-    tails_init_kernel<<<dim3(1), dim3(256), 0, s>>>(p.offsets, p.G, p.M, p.tails);
+    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails);
   }
   if (pingpong && p.tails != nullptr) {
     if (swiglu) {
