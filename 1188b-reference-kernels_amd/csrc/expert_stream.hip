@@ -402,7 +402,7 @@ __global__ __launch_bounds__(512) void expert_stream_kernel(GemmArgs p) {
   if (p.tails != nullptr) {
     // Only if every group is short; otherwise the ping-pong kernel that follows takes them all, and needs its list.
     if (tiles[0] > 0) {
-      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails);
+      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails, 0);
       return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) no_tails(p.tails);
@@ -412,11 +412,12 @@ __global__ __launch_bounds__(512) void expert_stream_kernel(GemmArgs p) {
   if (plan.row_tiles == 0) return;
   {
     // Whole rounds of the workgroups, as many as units of the full width need; no unit narrower than a slab.
-    constexpr int64_t kMax = kSwiglu ? kBRows / 32 : kBRows / 16;
-    const int64_t c16 = (p.ncols + 15) / 16, P = gridDim.x;
-    const int64_t need = plan.row_tiles * ((c16 + kMax - 1) / kMax);
+    // (32 bits: at most 64 rows per group on average, 4096 groups and 2^19 columns.)
+    constexpr uint32_t kMax = kSwiglu ? kBRows / 32 : kBRows / 16;
+    const uint32_t c16 = static_cast<uint32_t>(p.ncols + 15) / 16, P = gridDim.x, n = static_cast<uint32_t>(plan.row_tiles);
+    const uint32_t need = n * ((c16 + kMax - 1) / kMax);
     plan.c16 = static_cast<int>(c16);
-    plan.units = static_cast<int>(min((need + P - 1) / P * P, plan.row_tiles * c16));
+    plan.units = static_cast<int>(min((need + P - 1) / P * P, n * c16));
   }
   if (tiles[0] > 0) run_class<128, kSwiglu, kGather>(p, plan, role, lds, first, 0);
   if (tiles[1] > 0) run_class<64, kSwiglu, kGather>(p, plan, role, lds, first, tiles[0]);

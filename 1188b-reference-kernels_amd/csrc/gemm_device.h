@@ -142,18 +142,24 @@ __device__ __forceinline__ int main_row_tiles(int m) { return (m + 255 - kTailMa
 // The list, by one wavefront: each lane counts the tails of its chunk of
 // groups, an exclusive scan over the lanes gives the chunk's first list
 // position, then each lane lists its chunk's tail groups. Group g is rows
-// offsets[g] .. offsets[g + 1] - 1, clamped to [0, M].
-__device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
+// offsets[g] .. offsets[g + 1] - 1, clamped to [0, M]. If no group has more
+// than `shorts` rows, another kernel computes them all (kTailNone).
+__device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails, int64_t shorts) {
   const int lane = lane_id();
   const int64_t per = (G + kWave - 1) / kWave;
   const int64_t g0 = min(G, lane * per), g1 = min(G, g0 + per);
-  auto tail_at = [&](int64_t g) {
+  auto rows = [&](int64_t g) {
     const int64_t lo = min(max(static_cast<int64_t>(offsets[g]), int64_t(0)), M);
-    const int64_t hi = min(max(static_cast<int64_t>(offsets[g + 1]), lo), M);
-    return has_tail(hi - lo);
+    return min(max(static_cast<int64_t>(offsets[g + 1]), lo), M) - lo;
   };
   int n = 0;
-  for (int64_t g = g0; g < g1; ++g) n += tail_at(g) ? 1 : 0;
+  bool longer = false;
+  for (int64_t g = g0; g < g1; ++g) {
+    const int64_t m = rows(g);
+    n += has_tail(m) ? 1 : 0;
+    longer |= m > shorts;
+  }
+  const bool any_longer = __ballot(longer) != 0;
   int pos = n;
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -162,12 +168,12 @@ __device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, in
   }
   if (lane == kWave - 1) {
     tails[kTailCount] = pos;
-    tails[kTailNone] = 0;
+    tails[kTailNone] = any_longer ? 0 : 1;
     tails[kTailCtr] = 0;
   }
   pos -= n;
   for (int64_t g = g0; g < g1; ++g) {
-    if (tail_at(g)) tails[kTailList + pos++] = static_cast<int>(g);
+    if (has_tail(rows(g))) tails[kTailList + pos++] = static_cast<int>(g);
   }
 }
 
@@ -180,8 +186,9 @@ __device__ __forceinline__ void no_tails(int *tails) {
 
 namespace {
 
-__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
-  tails_list(offsets, G, M, tails);
+__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails,
+                                                       int64_t shorts) {
+  tails_list(offsets, G, M, tails, shorts);
 }
 
 }  // namespace

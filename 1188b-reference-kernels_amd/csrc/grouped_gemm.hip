@@ -1520,28 +1520,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_fwd128_kernel(GemmArgs p) {
   const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
   const int m32 = static_cast<int>(p.M), g_count = static_cast<int>(p.G);
   const int ntl = static_cast<int>((N + kTN - 1) / kTN);
-  if (p.tails != nullptr) {
-    // Only if every group fits one row tile; otherwise the ping-pong kernel that follows takes them all, and
-    // needs its list.
-    bool longer = false;
-    for (int g = threadIdx.x; g < g_count; g += 512) {
-      const int lo = min(max(p.offsets[g], 0), m32);
-      longer |= min(max(p.offsets[g + 1], lo), m32) - lo > kTM;
-    }
-    volatile int *any = reinterpret_cast<volatile int *>(smem);
-    const bool wave_any = __ballot(longer) != 0;
-    if (lane == 0) any[wave] = wave_any;
-    __syncthreads();
-    int found = 0;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) found |= any[w];
-    __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(found)) {
-      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails);
-      return;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) no_tails(p.tails);
-  }
+  // Only if every group fits one row tile, where a list was made first; otherwise the ping-pong kernel takes them all.
+  if (p.tails != nullptr && ld_inv(p.tails, kTailNone) == 0) return;
 
   // ---- tile walker (every wavefront walks the same tiles): group by group, row tile-major
   struct Tile {
@@ -1782,6 +1762,15 @@ int fwd128_nb(int64_t M_total, int64_t N, int64_t G, int64_t P) {
   return best;
 }
 
+// Whether those tiles fill their rounds to 2%, and are wider than the stream's 128 columns or take one round only.
+// Then the 128-row kernel is as fast as the stream or faster (us, it and the stream: 40 groups of 16 rows, K 8192, N
+// 5120: 535, 544; one round: 8 groups of 11 rows, K 1344, N 6096: 24, 26; 4 of 25, K 1024, N 8192: 14, 17).
+bool fwd128_even(int64_t M_total, int64_t N, int64_t G, int64_t P) {
+  const int nb = fwd128_nb(M_total, N, G, P);
+  const int64_t tn = 32 * nb, rounds = moe::ceil_div(G * moe::ceil_div(N, tn), P);
+  return (nb > 4 || rounds == 1) && rounds * P * tn * 50 <= 51 * G * N;
+}
+
 int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows, const int32_t *a_rows,
                         int64_t M_total, int64_t K, const moe_bf16_t *w, int64_t G, int64_t N,
                         const int32_t *group_offsets, int epilogue, moe_bf16_t *out, void *workspace,
@@ -1840,8 +1829,12 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
   p.tails = nullptr;
   p.split_tiles = p.split_ways = p.split_steps = 0;
   p.planes = nullptr;
-  // A few rows per group: the stream of the weights.
-  if (pingpong && M_total <= kStreamRows * G && ncols < (int64_t(1) << 19)) {
+  const int64_t P = std::max<int64_t>(8, num_cus() / 8 * 8);
+  const bool in_place = MOE_GEMM_FWD128 && !swiglu && !gather;
+  // A few rows per group: the stream of the weights (with 8 rows or more on average most groups have some, and the
+  // rounds of the 128-row kernel can be told here).
+  if (pingpong && M_total <= kStreamRows * G && ncols < (int64_t(1) << 19) &&
+      !(in_place && M_total >= 8 * G && fwd128_even(M_total, N, G, P))) {
     launch_expert_stream(p, swiglu, gather, s);
     return check_launch(fn);
   }
@@ -1849,18 +1842,20 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
                        is_aligned(workspace, 256);
   // Groups of at most 128 rows on average: the kernels for short groups, where the groups are short. With a workspace
   // they look at the groups first and leave a skewed split, in which a few groups hold most of the rows, to the
-  // ping-pong kernel, whose tail list the first launch then makes (a few us for the launch that finds nothing to do).
+  // ping-pong kernel, whose tail list the launch that looks makes (a few us for the launches that find nothing to do).
   // Plain, 1023 tokens over 64 experts top-8 (K 2048, N 7168): 588 us in 128-row tiles throughout, 426 us this way;
   // 40 even groups of 102 rows (K 8192, N 5120): 664 us in 128-row tiles, 735 in the ping-pong kernel's. SwiGLU and
   // gather, 64 even groups of 48 and 64 rows (K 7168, N 4096): 633 and 636 us in the ping-pong kernel's tail tiles,
   // 574 and 603 streamed; of 100 rows 649 against 691.
   bool list_made = false;
   if (pingpong && M_total <= 128 * G) {
-    const bool look = tail_ws && M_total > 128;  // (otherwise no group has more)
+    // (No group has more than 128 rows if there are no more in all; and below 512 MB of weights, some 90 us, the second
+    // launch costs what it can save.)
+    const bool look = tail_ws && M_total > 128 && (!in_place || G * N * K >= int64_t(1) << 28);
     if (look) p.tails = static_cast<int *>(workspace);
-    if (MOE_GEMM_FWD128 && !swiglu && !gather) {
+    if (in_place) {
       // Plain epilogue, A rows in place: 128-row tiles with their own loading wavefronts.
-      const int64_t P = std::max<int64_t>(8, num_cus() / 8 * 8);
+      if (look) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails, 128);
       switch (MOE_GEMM_FWD128_NB ? MOE_GEMM_FWD128_NB : fwd128_nb(M_total, N, G, P)) {
         case 4: grouped_gemm_fwd128_kernel<4><<<dim3(P), dim3(512), 0, s>>>(p); break;
         case 5: grouped_gemm_fwd128_kernel<5><<<dim3(P), dim3(512), 0, s>>>(p); break;
@@ -1911,7 +1906,7 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
   }
   if (tail_ws) {
     p.tails = static_cast<int *>(workspace);
-    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails);
+    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails, 0);
   }
   if (pingpong && p.tails != nullptr) {
     if (swiglu) {

@@ -77,3 +77,19 @@ def test_choice_by_group_sizes(pkg, dev, sizes, swiglu, gather):
     for _ in range(2):  # the second call finds the first one's list
         _same(call(workspace=ws), drained, "with a workspace")
     _same(call(workspace=torch.empty(0, dtype=torch.uint8, device=dev)), drained, "without one")
+
+
+@pytest.mark.parametrize("sizes", [[128, 40, 0, 90, 64, 100, 30], [129, 40, 0, 90, 64, 100, 30], [700, 3, 0, 9, 130, 1, 2]])
+def test_choice_by_group_sizes_plain_large(pkg, dev, sizes):
+    # A rows in place, plain: the launch looks at the groups from 2^28 weights on.
+    M, G, N, K = sum(sizes), len(sizes), 8192, 4736
+    assert 32 * G < M <= 128 * G and G * N * K >= 1 << 28
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.stack([(torch.randn(N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16) for _ in range(G)])
+    offs = pkg.ops.group_offsets_from_splits(sizes, dev)
+    buf = torch.full((M * N + 16,), float("nan"), dtype=torch.bfloat16, device=dev)
+    drained = pkg.ops.grouped_gemm(x, w, offs, out=buf[1:1 + M * N].view(M, N))
+    ws = torch.full((512,), 0xAB, dtype=torch.uint8, device=dev)
+    for _ in range(2):
+        _same(pkg.ops.grouped_gemm(x, w, offs, workspace=ws), drained, "with a workspace")
