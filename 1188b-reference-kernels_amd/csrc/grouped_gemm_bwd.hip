@@ -27,7 +27,7 @@
 // reduction step of 64 and an LDS ring filled by buffer_load ... lds ahead of
 // the MFMAs:
 //   * grouped_gemm_bwd_pipe_kernel (every 256 x 256 tile: dgrad with groups
-//     above ~160 rows, wgrad, the tf32 router GEMMs): the forward pipelined
+//     above ~160 rows, wgrad, the tf32 router dgrad's split form): the forward pipelined
 //     kernel's shape, v_mfma_f32_16x16x32_bf16 on 2 x 2 waves of 128 x 128,
 //     two stages, tiles chained without draining the pipeline, epilogue from
 //     registers; described above the kernel;
@@ -52,6 +52,7 @@
 #include <type_traits>
 
 #include "gemm_device.h"
+#include "tf32_device.h"
 
 namespace moe {
 namespace {
@@ -140,24 +141,6 @@ __device__ __forceinline__ bf16x8 read_rm_frag_rows(uint32_t addr) {
 }
 // The same with 256-column tiles (kRMRow-byte rows).
 __device__ __forceinline__ bf16x8 read_rm_frag(uint32_t addr) { return read_rm_frag_rows<kRMRow>(addr); }
-
-// One 16 x 16 x 32 MFMA on 16-bit operands: bf16, or fp16 (kF16: the tf32 router GEMMs' scaled operands,
-// the same bit layout in LDS and registers).
-template <bool kF16>
-__device__ __forceinline__ f32x4_t mma16(bf16x8 a, bf16x8 b, f32x4_t c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (kF16) {
-    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-#else
-  (void)a;
-  (void)b;
-  return c;
-#endif
-}
 
 // The 128-row dgrad kernel (groups of at most ~160 rows, reductions that are
 // not whole steps): 1 x 4 waves of 128 x 64, a three-stage ring (the stream of
@@ -598,7 +581,7 @@ __global__ __launch_bounds__(256, kTN == 128 ? 2 : 1) void grouped_gemm_dgrad128
 
 // ---- pipelined 256 x 256 kernel ---------------------------------------------
 // The kernel the host runs for every 256-row tile (dgrad with groups above
-// ~160 rows, wgrad, and the tf32 router GEMMs): the forward pipelined kernel's
+// ~160 rows, wgrad, and the tf32 router dgrad's split form): the forward pipelined kernel's
 // shape with reduction-major operands.
 //   * v_mfma_f32_16x16x32_bf16, 8 x 8 blocks of 16 x 16 per wave (the board
 //     holds a higher clock under it than under the 32 x 32 x 16 form);
@@ -627,9 +610,8 @@ __device__ __forceinline__ int rm16_swz(int krow) { return ((krow & 3) << 2) | (
 // [M, K] of out (at the same row indices).
 // kOrder (wgrad): the tiles take the groups in the order p.order lists them
 // (largest first, from group_order_kernel) instead of by index.
-template <bool kWgrad, int kOut, bool kSplit = false, bool kOrder = false, bool kF16 = false>
+template <bool kWgrad, int kOut, bool kSplit = false, bool kOrder = false>
 __global__ __launch_bounds__(256) void grouped_gemm_bwd_pipe_kernel(BwdArgs p) {
-  static_assert(!kF16 || (kWgrad && kOut == 1), "fp16 operands: the tf32 router wgrad (fp32 planes)");
   static_assert(!kSplit || (!kWgrad && kOut == 1), "the split is a dgrad with fp32 planes");
   static_assert(!kOrder || kWgrad, "the group order is a wgrad schedule");
   constexpr int kBM = 256;
@@ -889,7 +871,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_bwd_pipe_kernel(BwdArgs p) {
     for (int j = 0; j < kNI; ++j) {
 #pragma unroll
       for (int i = 4; i < 8; ++i) {
-        acc[i][j] = mma16<kF16>(fb[1][j], fa[1][i], acc[i][j]);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
       }
       fb[1][j] = rm_frag(base_b, x, j, 1);
       if (j < 4) {
@@ -907,7 +889,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_bwd_pipe_kernel(BwdArgs p) {
     for (int i = 4 * ih; i < 4 * ih + 4; ++i)
 #pragma unroll
       for (int j = 0; j < kNI; ++j)
-        acc[i][j] = mma16<kF16>(fb[ks][j], fa[ks][i], zero ? f32x4{} : acc[i][j]);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[ks][j], fa[ks][i], zero ? f32x4{} : acc[i][j], 0, 0, 0);
   };
 
   // Epilogue of tile t from the accumulators: register r of lane l in block
@@ -1640,7 +1622,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_wgrad_sweep_kernel(BwdArgs p
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          acc[i][j] = mma16<false>(fb[j], fa[i], ks == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], ks == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
     }
   };
   // Epilogue: register r of lane l in block (i, j) holds dw row wn * 64 + i * 16 + l % 16 and column
@@ -1770,11 +1752,11 @@ SweepPlan sweep_plan(int64_t N, int64_t K, int64_t G, int64_t cus) {
   return best;
 }
 
-template <bool kWgrad, int kOut = 0, bool kSplit = false, bool kOrder = false, bool kF16 = false>
+template <bool kWgrad, int kOut = 0, bool kSplit = false, bool kOrder = false>
 void launch_pipe(const BwdArgs &p, int64_t max_tiles, hipStream_t s) {
   int64_t grid = std::min<int64_t>(num_cus(), max_tiles);
   grid = std::max<int64_t>(8, (grid + 7) / 8 * 8);
-  grouped_gemm_bwd_pipe_kernel<kWgrad, kOut, kSplit, kOrder, kF16><<<dim3(grid), dim3(256), 0, s>>>(p);
+  grouped_gemm_bwd_pipe_kernel<kWgrad, kOut, kSplit, kOrder><<<dim3(grid), dim3(256), 0, s>>>(p);
 }
 
 #ifndef MOE_GEMM_BWD_PINGPONG
@@ -1862,12 +1844,6 @@ void launch_dgrad128(const BwdArgs &p, int64_t max_tiles, hipStream_t s) {
 // a b = hi_a hi_b + hi_a lo_b + lo_a hi_b + lo_a lo_b with the last term,
 // below 2^-16 |a b|, dropped: three bf16 products per tf32 product, each exact
 // in the fp32 accumulator.
-__device__ __forceinline__ uint32_t tf32_rne_bits(uint32_t b) {
-  const uint32_t low = b & 0x1FFFu, lsb = (b >> 13) & 1u;
-  const uint32_t add = (low == 0x1000u && lsb == 0u) ? 0u : 0x1000u;
-  return (b + add) & 0xFFFFE000u;
-}
-
 // src fp32 [rows, cols] (cols % 4 == 0) -> hi (and a second copy hi2) and lo
 // bf16 planes with their own row strides (null planes are skipped).
 struct SplitArgs {
@@ -1908,29 +1884,7 @@ void launch_split(const SplitArgs &a, hipStream_t s) {
   tf32_split_kernel<<<dim3(grid), dim3(256), 0, s>>>(a);
 }
 
-// ---- tf32 wgrad on the fp16 matrix cores --------------------------------
-// A tf32 value has 11 significant bits, as many as fp16. Scaled by the power of
-// two 2^e that brings the largest magnitude of its column into [2^14, 2^15),
-// every tf32-rounded value of the column is an fp16 value, exactly unless it
-// lies 2^29 or more below that largest one (it then rounds to an fp16
-// subnormal: an error below 2^-38 of the column's largest magnitude). The
-// product of two fp16 values is exact in fp32, so one fp16 MFMA replaces the
-// three bf16 products of the hi/lo split, and the fp32 sums are scaled back by
-// 2^-(e_row + e_col) (exact) when the reduction planes are added. The scale
-// comes from the largest finite magnitude (Inf and NaN entries stay Inf and
-// NaN when scaled, so every finite value still converts exactly); a column
-// with no finite nonzero value keeps scale 1.
-__device__ __forceinline__ float finite_abs(float x) {
-  const float a = fabsf(x);
-  return a < __builtin_huge_valf() ? a : 0.f;  // Inf and NaN -> 0
-}
-__device__ __forceinline__ int scale_exp(float mx) {
-  if (!(mx > 0.f) || !(mx < __builtin_huge_valf())) return 0;
-  int e = 0;
-  (void)__builtin_frexpf(mx, &e);  // mx = f 2^e, f in [0.5, 1)
-  return 15 - e;                   // mx 2^(15 - e) in [2^14, 2^15)
-}
-
+// ---- scaled fp16 copies (tf32_device.h) ----------------------------------
 // Largest finite magnitude per column over a slab of rows: block (x, y) covers cg
 // groups of 4 columns from x 4 cg and rows y rps .. + rps - 1, its threads
 // split over the groups (t % cg) and 256 / cg interleaved row phases (t / cg,
@@ -2075,33 +2029,6 @@ __global__ __launch_bounds__(256) void tf32_to_f16_cols_kernel(const float *src,
     }
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     *reinterpret_cast<u32x2 *>(dst + r * C + c) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-  }
-}
-
-// out[n][k] = 2^-(row_exp[n] + col_exp[k]) sum over s of part[s][n][k], s ascending (K % 4 == 0).
-__global__ __launch_bounds__(256) void sum_planes_scaled_kernel(const float *part, int planes, int64_t N, int64_t K,
-                                                                const int32_t *row_exp, const int32_t *col_exp, float *out) {
-  const int64_t n = N * K;
-  const int64_t q = n / 4, qk = K / 4;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < q; i += stride) {
-    u32x4 a = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(part) + i);
-    float x = __uint_as_float(a.x), y = __uint_as_float(a.y), z = __uint_as_float(a.z), w = __uint_as_float(a.w);
-    for (int s = 1; s < planes; ++s) {
-      const u32x4 b = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(part + s * n) + i);
-      x += __uint_as_float(b.x);
-      y += __uint_as_float(b.y);
-      z += __uint_as_float(b.z);
-      w += __uint_as_float(b.w);
-    }
-    const int64_t row = i / qk, col = (i - row * qk) * 4;
-    const int er = row_exp[row];
-    const int4 ec = *reinterpret_cast<const int4 *>(col_exp + col);
-    x = __builtin_ldexpf(x, -(er + ec.x));
-    y = __builtin_ldexpf(y, -(er + ec.y));
-    z = __builtin_ldexpf(z, -(er + ec.z));
-    w = __builtin_ldexpf(w, -(er + ec.w));
-    *(reinterpret_cast<u32x4 *>(out) + i) = u32x4{__float_as_uint(x), __float_as_uint(y), __float_as_uint(z), __float_as_uint(w)};
   }
 }
 
@@ -2519,62 +2446,42 @@ int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const 
 
 namespace {
 
-// Reduction split of the tf32 router wgrad: the output has few tiles
-// (case31: 2 x 32 for 256 CUs), so the M rows are cut into uniform chunks run
-// as groups of one launch, every chunk writing its own fp32 partial
-// [N, K]; a last pass adds the partials in chunk order.
-struct WgradPlan {
-  int64_t s;  // chunks (1 = no split)
-  int64_t c;  // rows per chunk
-};
-
-WgradPlan wgrad_plan(int64_t rows, int64_t N, int64_t K) {
-  WgradPlan pl{1, rows};
-  const int64_t tiles = moe::ceil_div(N, 256) * moe::ceil_div(K, 256);
-  if (rows == 0 || tiles >= 256) return pl;
-  // one round of work items on 256 CUs (case31: 4 chunks of 4096 rows, 0.403-0.406 -> 0.391-0.392 ms against 8
-  // chunks in two rounds: one tile epilogue per CU and half the planes; 16 chunks: 0.446-0.450)
-  int64_t s = std::min<int64_t>(moe::ceil_div(256, tiles), std::max<int64_t>(1, rows / 512));
-  s = std::max<int64_t>(1, std::min<int64_t>(s, 64));
-  if (s == 1) return pl;
-  // Chunks are multiples of 64 rows (whole reduction steps).
-  pl.c = moe::ceil_div(moe::ceil_div(rows, s), 64) * 64;
-  pl.s = moe::ceil_div(rows, pl.c);
-  return pl;
-}
-
-// Workspace of the tf32 wgrad (byte offsets, each 256-byte aligned): the fp16
-// copies of grad_output [M, N] and inp [M, K], the scale exponents of their
-// columns, the column-max slabs, and the fp32 planes of the reduction chunks
-// (one plane at least: the scale is undone where the planes are added).
+// Workspace of the tf32 wgrad (byte offsets, each 256-byte aligned): the transposed fp16 copy of grad_output, its
+// scale exponents, its column-max slabs, and the fp32 planes of the reduction chunks (none for one chunk). Its size is
+// never below `agreed`, what callers that sized their workspaces once were told: fp16 copies of both operands, both
+// operands' exponents and column-max slabs, and the planes of chunks of 512 rows or more.
 struct WgradTf32Layout {
-  WgradPlan pl;
-  moe::ColmaxPlan ca, cb;
-  size_t a16, b16, row_exp, col_exp, part_a, part_b, planes, total;
+  moe::RouterWgradPlan pl;
+  moe::ColmaxPlan ca;
+  size_t rows, exp, part, planes, total;
 };
 WgradTf32Layout wgrad_tf32_layout(int64_t M, int64_t N, int64_t K) {
   using moe::align_up;
   WgradTf32Layout l;
-  l.pl = wgrad_plan(M, N, K);
+  l.pl = moe::router_wgrad_plan(M, N, K);
   l.ca = moe::colmax_plan(M, N);
-  l.cb = moe::colmax_plan(M, K);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
     off += align_up(bytes);
     return at;
   };
-  l.a16 = take(static_cast<size_t>(M) * N * 2);
-  l.b16 = take(static_cast<size_t>(M) * K * 2);
-  l.row_exp = take(static_cast<size_t>(N) * 4);
-  l.col_exp = take(static_cast<size_t>(K) * 4);
-  l.part_a = take(static_cast<size_t>(l.ca.S) * N * 4);
-  l.part_b = take(static_cast<size_t>(l.cb.S) * K * 4);
-  l.planes = take(static_cast<size_t>(l.pl.s) * N * K * 4);
-  l.total = off;
+  l.rows = take(static_cast<size_t>(moe::ceil_div(M, 64) * 64) * N * 2);
+  l.exp = take(static_cast<size_t>(N) * 4);
+  l.part = take(static_cast<size_t>(l.ca.S) * N * 4);
+  l.planes = take(l.pl.s > 1 ? static_cast<size_t>(l.pl.s) * N * K * 4 : 0);
+  const int64_t tiles = moe::ceil_div(N, 256) * moe::ceil_div(K, 256);
+  int64_t chunks = 1;
+  if (M > 0 && tiles > 0 && tiles < 256) {
+    chunks = std::min<int64_t>({moe::ceil_div(256, tiles), std::max<int64_t>(1, M / 512), 64});
+    if (chunks > 1) chunks = moe::ceil_div(M, moe::ceil_div(moe::ceil_div(M, chunks), 64) * 64);
+  }
+  const size_t agreed = align_up(static_cast<size_t>(M) * N * 2) + align_up(static_cast<size_t>(M) * K * 2) + align_up(static_cast<size_t>(N) * 4) +
+                        align_up(static_cast<size_t>(K) * 4) + align_up(static_cast<size_t>(l.ca.S) * N * 4) +
+                        align_up(static_cast<size_t>(moe::colmax_plan(M, K).S) * K * 4) + align_up(static_cast<size_t>(chunks) * N * K * 4);
+  l.total = std::max(off, agreed);
   return l;
 }
-
 
 }  // namespace
 
@@ -2611,50 +2518,14 @@ int moe_router_wgrad_tf32(const float *grad_output, int64_t M, int64_t N, const 
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *w = static_cast<char *>(workspace);
-  uint16_t *a16 = reinterpret_cast<uint16_t *>(w + l.a16);
-  uint16_t *b16 = reinterpret_cast<uint16_t *>(w + l.b16);
-  int32_t *row_exp = reinterpret_cast<int32_t *>(w + l.row_exp);
-  int32_t *col_exp = reinterpret_cast<int32_t *>(w + l.col_exp);
-  float *part_a = reinterpret_cast<float *>(w + l.part_a);
-  float *part_b = reinterpret_cast<float *>(w + l.part_b);
-  float *planes = reinterpret_cast<float *>(w + l.planes);
-  // Scale exponents of grad_output's columns (dw rows) and inp's columns (dw columns), then the fp16 copies.
+  uint16_t *rows = reinterpret_cast<uint16_t *>(w + l.rows);
+  int32_t *exp = reinterpret_cast<int32_t *>(w + l.exp);
+  float *part = reinterpret_cast<float *>(w + l.part);
+  // grad_output's column maxima (dw rows), its scaled transpose, then the GEMM, which scales inp on the way.
   colmax_partial_kernel<<<dim3(static_cast<uint32_t>(l.ca.xb), static_cast<uint32_t>(l.ca.S)), dim3(256), 0, s>>>(
-      grad_output, M, N, l.ca.rps, l.ca.cg, part_a);
-  colmax_partial_kernel<<<dim3(static_cast<uint32_t>(l.cb.xb), static_cast<uint32_t>(l.cb.S)), dim3(256), 0, s>>>(
-      inp, M, K, l.cb.rps, l.cb.cg, part_b);
-  colmax_final_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N, 256))), dim3(256), 0, s>>>(part_a, static_cast<int>(l.ca.S), N,
-                                                                                          row_exp, nullptr);
-  colmax_final_kernel<<<dim3(static_cast<uint32_t>(ceil_div(K, 256))), dim3(256), 0, s>>>(part_b, static_cast<int>(l.cb.S), K,
-                                                                                          col_exp, nullptr);
-  if (M > 0) {
-    const int64_t ga = std::max<int64_t>(1, std::min<int64_t>(ceil_div(M * N / 4, 256), 8192));
-    const int64_t gb = std::max<int64_t>(1, std::min<int64_t>(ceil_div(M * K / 4, 256), 8192));
-    tf32_to_f16_cols_kernel<<<dim3(static_cast<uint32_t>(ga)), dim3(256), 0, s>>>(grad_output, M, N, row_exp, a16);
-    tf32_to_f16_cols_kernel<<<dim3(static_cast<uint32_t>(gb)), dim3(256), 0, s>>>(inp, M, K, col_exp, b16);
-  }
-  if (int rc = check_launch(fn)) return rc;
-  // dw planes over the reduction chunks (fp16 MFMA, exact products, fp32 sums), then their sum scaled back.
-  BwdArgs p;
-  p.a = a16;
-  p.b = b16;
-  p.offsets = nullptr;
-  p.out = planes;
-  p.M = M;
-  p.N = N;
-  p.K = K;
-  p.G = l.pl.s;
-  p.ntiles = ceil_div(K, kBN);
-  p.chunk = l.pl.c;
-  p.kchunk = 0;
-  p.order = nullptr;
-  p.order_rows = nullptr;
-  p.tails = nullptr;
-  launch_pipe<true, 1, false, false, true>(p, ceil_div(N, 256) * p.ntiles * p.G, s);
-  const int64_t q = N * K / 4;
-  const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(ceil_div(q, 256), 4096));
-  sum_planes_scaled_kernel<<<dim3(static_cast<uint32_t>(grid)), dim3(256), 0, s>>>(planes, static_cast<int>(l.pl.s), N, K,
-                                                                                   row_exp, col_exp, grad_weight);
+      grad_output, M, N, l.ca.rps, l.ca.cg, part);
+  launch_router_wgrad_rows(grad_output, M, N, part, static_cast<int>(l.ca.S), rows, exp, s);
+  launch_router_wgrad(l.pl, rows, exp, inp, M, N, K, reinterpret_cast<float *>(w + l.planes), grad_weight, s);
   return check_launch(fn);
 }
 

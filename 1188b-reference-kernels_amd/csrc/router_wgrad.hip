@@ -1,0 +1,350 @@
+// tf32 router weight gradient: grad_weight [N, K] = tf32(grad_output [M, N])^T tf32(inp [M, K]), fp32 in and out, on
+// the fp16 matrix cores (tf32_device.h).
+//
+// inp is the large operand (M x K fp32, 537 MB at 16384 x 8192) and is read once, straight from memory into the
+// registers of the wavefront that multiplies it:
+//   * a wavefront owns 32 columns of inp and all N (<= 320 a row tile) rows of the result. In the B operand of
+//     v_mfma_f32_16x16x32_f16 lane l holds 8 consecutive reduction rows 8 (l / 16) .. + 7 of column l % 16, so a lane that
+//     loads two neighbouring columns of those 8 rows (8 bytes each, 128 contiguous bytes per row over 16 lanes) holds
+//     the fragments of two blocks, the even columns and the odd ones: no LDS, no transpose, no fp16 copy in memory;
+//   * the columns' scales are found on the way: a lane compares its magnitudes with the largest its column's scale
+//     takes (one ballot per 32 rows); only when one exceeds it (in the first rows, then rarely: the scale leaves a
+//     factor of 8) the column's maximum is formed across the lanes, and the sums so far, whose column is the lane's
+//     own, are multiplied by the change, a power of two;
+//   * the small operand (grad_output, transposed and scaled in fp16 by a kernel before) comes through a ring of three
+//     LDS stages of 64 reduction rows, shared by the 8 wavefronts (256 columns);
+//   * M is cut into chunks so that there is a unit for every CU; the units of one XCD share a chunk, whose part of the
+//     small operand then stays in its L2. The planes of the chunks are added in order.
+// Measured (MI355X, 16384 x 320 x 8192, us): 395 -> 175 for the whole call; the GEMM 124-134 (4.0-4.3 TB/s of inp), the
+// planes' sum 16, grad_output's maxima and copy 17. Before: column maxima of inp 90, its fp16 copy 180, a GEMM on the
+// copies 143, the sum 10. 16384 x 64 x 7168: 307 -> 136; 4096 x 128 x 7168: 98 -> 74; 100 x 64 x 7168: 39 -> 19.
+#include <algorithm>
+#include <type_traits>
+
+#include "gemm_device.h"
+#include "tf32_device.h"
+
+namespace moe {
+namespace {
+
+using namespace gemm;
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+
+constexpr int kColsWave = 32, kColsTile = 256;
+constexpr int kRowB = kBK * 2;  // 128 bytes: one row of the small operand in a stage
+constexpr int64_t kWideK = int64_t(1) << 22;
+constexpr int kHeadroom = 3;    // a new scale puts the largest magnitude into [2^11, 2^12)
+
+__device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
+
+struct WgradArgs {
+  const uint16_t *rows;  // [N, M64] fp16
+  const int32_t *exp;    // [N]
+  const float *inp;      // [M, K]
+  float *out;            // planes [s, N, K]
+  int64_t M, M64, N, K;
+  int64_t chunk;         // reduction rows of a chunk
+  int col_tiles, row_tiles, units;
+};
+
+// kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets).
+template <int kMI, bool kWide>
+__global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
+  constexpr int kStage = kMI * 16 * kRowB;
+  constexpr int kSlots = 3;
+  constexpr int kDma = kMI * 2 / 8;  // 1 KiB blocks per wavefront and stage
+  constexpr int kBufs = 3;           // halves (32 reduction rows) of inp in registers
+  static_assert(kMI % 4 == 0 && kSlots * kStage <= 160 * 1024, "stage");
+  __shared__ __attribute__((aligned(1024))) char smem[kSlots * kStage];
+  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char *)smem));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int c16 = lane & 15, q = lane >> 4;
+
+  // Units chunk by chunk, then column tile by column tile, the row tiles of one fastest (they read the same inp).
+  const int b = static_cast<int>(blockIdx.x), P = static_cast<int>(gridDim.x);
+  const int u = (b % 8) * (P / 8) + b / 8;
+  if (u >= p.units) return;
+  const int per_chunk = p.col_tiles * p.row_tiles;
+  const int chunk = u / per_chunk, tile = u - chunk * per_chunk;
+  const int ct = tile / p.row_tiles, n0 = (tile - ct * p.row_tiles) * kMI * 16;
+  const int64_t m0 = chunk * p.chunk, mrows = min(p.chunk, p.M - m0);
+  const int steps = static_cast<int>((mrows + kBK - 1) / kBK);
+  [[maybe_unused]] const int halves = 2 * steps;
+
+  // ---- the small operand: this wavefront's blocks wave + 8 j of 8 rows
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.rows + static_cast<int64_t>(n0) * p.M64 + m0,
+                                              static_cast<uint32_t>(((min<int64_t>(p.N - n0, kMI * 16) - 1) * p.M64 + p.M64 - m0) * 2));
+  int a_off[kDma];
+#pragma unroll
+  for (int j = 0; j < kDma; ++j) {
+    const int r = (wave + 8 * j) * 8 + (lane >> 3);
+    a_off[j] = n0 + r < p.N ? static_cast<int>(static_cast<uint32_t>(r) * static_cast<uint32_t>(p.M64 * 2) +
+                                               static_cast<uint32_t>(((lane & 7) ^ swz128(r)) << 4))
+                            : static_cast<int>(kNoAccess);
+  }
+  // Stage st into its slot; past the last one the last one again, into a slot that nothing reads any more.
+  auto dma = [&](int st) {
+    const uint32_t dst = lds + (st % kSlots) * kStage;
+    const int k = min(st, steps - 1) * kRowB;
+#pragma unroll
+    for (int j = 0; j < kDma; ++j) dma16b(ra, (lds_void *)(uintptr_t)(dst + (wave + 8 * j) * 1024), a_off[j], k);
+  };
+
+  // ---- inp: columns col, col + 1, rows 32 h + 8 q + r of half h; rows past the chunk and columns past K read zeros
+  const int col = ct * kColsTile + wave * kColsWave + 2 * c16;
+  const uint32_t ldb = static_cast<uint32_t>(p.K) * 4u;
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.inp + m0 * p.K, kWide ? 0u : static_cast<uint32_t>(mrows) * ldb);
+  const uint32_t b_off = col < p.K ? static_cast<uint32_t>(8 * q) * ldb + static_cast<uint32_t>(col) * 4u : kNoAccess;
+  u32x2 buf[kBufs][8];
+  auto load = [&](int h, u32x2 *dst) {
+    const uint32_t row = static_cast<uint32_t>(min(h, halves - 1)) * 32u;
+    if constexpr (kWide) {
+#pragma unroll
+      for (uint32_t r = 0; r < 8; ++r) {
+        const int64_t m = row + 8 * q + r;
+        dst[r] = m < mrows && col < p.K ? *reinterpret_cast<const u32x2 *>(p.inp + (m0 + m) * p.K + col) : u32x2{0u, 0u};
+      }
+      return;
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    // The rows' offsets are in the vector offset: the scalar one is not part of the range check.
+#pragma unroll
+    for (uint32_t r = 0; r < 8; ++r) dst[r] = __builtin_amdgcn_raw_buffer_load_b64(rb, static_cast<int>(b_off + (row + r) * ldb), 0, 2);
+#else
+    (void)row;
+    (void)b_off;
+    (void)rb;
+    (void)dst;
+#endif
+  };
+
+  f32x4 acc[kMI][2];
+#pragma unroll
+  for (int i = 0; i < kMI; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int e[2] = {0, 0};             // the columns' scale exponents
+  // Magnitudes below it fit the scale; at first the smallest there is, which only zeros are below.
+  float most[2] = {__uint_as_float(1u), __uint_as_float(1u)};
+  f16x8 fb[2];
+  auto convert = [&](const u32x2 *v) {
+    float mx[2] = {0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      mx[0] = fmaxf(mx[0], fabsf(__uint_as_float(v[r].x)));
+      mx[1] = fmaxf(mx[1], fabsf(__uint_as_float(v[r].y)));
+    }
+    if (__ballot(mx[0] >= most[0] || mx[1] >= most[1]) != 0) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float m = 0.f;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) m = fmaxf(m, finite_abs(__uint_as_float(j ? v[r].y : v[r].x)));
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        if (m >= most[j]) {
+          const int ne = scale_exp(m) - kHeadroom, d = ne - e[j];
+          e[j] = ne;
+          most[j] = __builtin_ldexpf(1.f, 15 - ne);
+#pragma unroll
+          for (int i = 0; i < kMI; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[i][j][t] = __builtin_ldexpf(acc[i][j][t], d);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        fb[j][r] = static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(j ? v[r].y : v[r].x)), e[j]));
+  };
+  // Half h of stage st (ks: which half of the stage).
+  auto multiply = [&](int slot, int ks) {
+    const uint32_t base = lds + slot * kStage;
+    const uint32_t at = base + c16 * kRowB + ((((ks << 2) | q) ^ swz128(c16)) << 4);  // 16 rows on: the same swizzle
+    f16x8 fa[2][2];
+    auto read = [&](int i, f16x8 *f) {
+      f[0] = *reinterpret_cast<const lds_f16x8 *>((uintptr_t)(at + i * 16 * kRowB));
+      f[1] = *reinterpret_cast<const lds_f16x8 *>((uintptr_t)(at + (i + 1) * 16 * kRowB));
+    };
+    read(0, fa[0]);
+#pragma unroll
+    for (int i = 0; i < kMI; i += 2) {
+      if (i + 2 < kMI) read(i + 2, fa[(i / 2 + 1) & 1]);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        acc[i + d][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[(i / 2) & 1][d], fb[0], acc[i + d][0], 0, 0, 0);
+        acc[i + d][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[(i / 2) & 1][d], fb[1], acc[i + d][1], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  if (steps > 0) {
+    dma(0);
+    dma(1);
+#pragma unroll
+    for (int h = 0; h < kBufs; ++h) load(h, buf[h]);
+    // One round: three stages, six halves, so that the slots and register sets are fixed. The wait before a stage's
+    // barrier leaves in flight what was issued after the loads of its first half, which follow its own DMA: the next
+    // stage's DMA and two halves' loads.
+    for (int st = 0; st < steps; st += 3) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        if (st + k < steps) {
+          wait_vm_n<kDma + 16>();
+          barrier();  // stage st + k has landed, and every wavefront is done with the stage before
+          dma(st + k + 2);
+          convert(buf[(2 * k) % 3]);
+          __builtin_amdgcn_sched_barrier(0);
+          load(2 * (st + k) + 3, buf[(2 * k) % 3]);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(k, 0);
+          convert(buf[(2 * k + 1) % 3]);
+          __builtin_amdgcn_sched_barrier(0);
+          load(2 * (st + k) + 4, buf[(2 * k + 1) % 3]);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(k, 1);
+        }
+      }
+    }
+    wait_dma();  // no LDS DMA outlives the workgroup
+  }
+
+  // acc[i][j] register t: row n0 + 16 i + 4 q + t, column col + j.
+  float *const out = p.out + (static_cast<int64_t>(chunk) * p.N + n0) * p.K;
+  if (col < p.K) {
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = i * 16 + q * 4 + t;
+        if (n0 + r < p.N) {
+          const int er = p.exp[n0 + r];
+          const u32x2 v = {__float_as_uint(__builtin_ldexpf(acc[i][0][t], -(er + e[0]))),
+                           __float_as_uint(__builtin_ldexpf(acc[i][1][t], -(er + e[1])))};
+          *reinterpret_cast<u32x2 *>(out + static_cast<int64_t>(r) * p.K + col) = v;
+        }
+      }
+    }
+  }
+}
+
+// Block (x, y): reduction rows 64 x .. + 63 and columns 64 y .. + 63 of grad_output, transposed through LDS. Each block
+// forms its columns' exponents from the slab maxima; those of x = 0 write them.
+__global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src, int64_t M, int64_t M64, int64_t N, const float *part,
+                                                                int slabs, uint16_t *dst, int32_t *exp) {
+  __shared__ int ex[64];
+  __shared__ float red[4][64];
+  __shared__ uint16_t tile[64][66];  // [column][row], padded against bank conflicts
+  const int t = threadIdx.x;
+  const int64_t m0 = static_cast<int64_t>(blockIdx.x) * 64, n0 = static_cast<int64_t>(blockIdx.y) * 64;
+  {
+    const int c = t & 63;
+    float m = 0.f;
+    if (n0 + c < N)
+      for (int s = t >> 6; s < slabs; s += 4) m = fmaxf(m, part[static_cast<int64_t>(s) * N + n0 + c]);
+    red[t >> 6][c] = m;
+  }
+  __syncthreads();
+  if (t < 64) {
+    const int e = scale_exp(fmaxf(fmaxf(red[0][t], red[1][t]), fmaxf(red[2][t], red[3][t])));
+    ex[t] = e;
+    if (blockIdx.x == 0 && n0 + t < N) exp[n0 + t] = e;
+  }
+  __syncthreads();
+  if (m0 >= M64) return;  // M = 0: the exponents only
+  {
+    const int c = (t & 15) * 4;  // N % 8 == 0: the four columns are all valid or all past N
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int r = (t >> 4) + 16 * k;
+      const bool in = m0 + r < M && n0 + c < N;
+      const u32x4 v = in ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + (m0 + r) * N + n0 + c)) : u32x4{0u, 0u, 0u, 0u};
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        tile[c + i][r] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(w[i])), ex[c + i])));
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = (t >> 3) + 32 * k, r = (t & 7) * 8;
+    if (n0 + c >= N) continue;
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const uint32_t *>(&tile[c][r + 2 * i]);
+    *reinterpret_cast<u32x4 *>(dst + (n0 + c) * M64 + m0 + r) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+}
+
+// out[i] = sum over s of planes[s][i], s ascending (n % 4 == 0).
+__global__ __launch_bounds__(256) void router_wgrad_sum_kernel(const float *planes, int s, int64_t n, float *out) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i * 4 >= n) return;
+  f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes) + i);
+  for (int k = 1; k < s; ++k) a += __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes + k * n) + i);
+  reinterpret_cast<f32x4 *>(out)[i] = a;
+}
+
+}  // namespace
+
+RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K) {
+  RouterWgradPlan pl;
+  pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 320));
+  const int64_t blocks = ceil_div(ceil_div(std::max<int64_t>(N, 1), pl.row_tiles), 16);
+  pl.mi = K >= kWideK || blocks <= 4 ? 4 : blocks <= 8 ? 8 : blocks <= 16 ? 16 : 20;
+  pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 16 * pl.mi));
+  const int64_t tiles = pl.row_tiles * std::max<int64_t>(1, ceil_div(K, kColsTile));
+  // A unit for every CU, of at least 128 rows; and a chunk of inp below 2 GiB (32-bit offsets).
+  int64_t s = std::min(ceil_div(256, tiles), std::max<int64_t>(1, M / 128));
+  if (K < kWideK) s = std::max(s, ceil_div(M * K, (int64_t(1) << 29) - 64 * K));
+  pl.c = std::max<int64_t>(1, ceil_div(ceil_div(M, s), kBK)) * kBK;
+  pl.s = std::max<int64_t>(1, ceil_div(M, pl.c));
+  return pl;
+}
+
+void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, const float *part, int slabs, uint16_t *rows, int32_t *exp,
+                              hipStream_t s) {
+  const int64_t M64 = ceil_div(M, 64) * 64;
+  router_wgrad_rows_kernel<<<dim3(static_cast<uint32_t>(std::max<int64_t>(1, M64 / 64)), static_cast<uint32_t>(ceil_div(N, 64))), dim3(256), 0,
+                             s>>>(grad_output, M, M64, N, part, slabs, rows, exp);
+}
+
+void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const int32_t *exp, const float *inp, int64_t M, int64_t N,
+                         int64_t K, float *planes, float *out, hipStream_t s) {
+  WgradArgs p;
+  p.rows = rows;
+  p.exp = exp;
+  p.inp = inp;
+  p.out = pl.s > 1 ? planes : out;
+  p.M = M;
+  p.M64 = ceil_div(M, 64) * 64;
+  p.N = N;
+  p.K = K;
+  p.chunk = pl.c;
+  p.col_tiles = static_cast<int>(ceil_div(K, kColsTile));
+  p.row_tiles = static_cast<int>(pl.row_tiles);
+  const int64_t units = pl.s * p.col_tiles * pl.row_tiles;
+  p.units = static_cast<int>(units);
+  const dim3 grid(static_cast<uint32_t>((units + 7) / 8 * 8)), block(512);
+  if (K >= kWideK) {
+    router_wgrad_kernel<4, true><<<grid, block, 0, s>>>(p);
+  } else {
+    switch (pl.mi) {
+      case 4: router_wgrad_kernel<4, false><<<grid, block, 0, s>>>(p); break;
+      case 8: router_wgrad_kernel<8, false><<<grid, block, 0, s>>>(p); break;
+      case 16: router_wgrad_kernel<16, false><<<grid, block, 0, s>>>(p); break;
+      default: router_wgrad_kernel<20, false><<<grid, block, 0, s>>>(p); break;
+    }
+  }
+  if (pl.s > 1) {
+    router_wgrad_sum_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N * K / 4, 256))), dim3(256), 0, s>>>(planes, static_cast<int>(pl.s), N * K, out);
+  }
+}
+
+}  // namespace moe

@@ -407,26 +407,28 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  * operands rounded to tf32 (round_tf32_rne, :51-58), products accumulated in
  * fp32, fp32 out.
  *   Both run on the fp16 matrix cores: a tf32 value has fp16's 11 significant
- *     bits; each operand row or column along which the sum runs is scaled by
- *     the power of two that brings its largest magnitude into [2^14, 2^15),
- *     so its values are fp16 values (exactly, unless 2^29 or more below that
- *     largest one: then within 2^-38 of it), the products are exact in fp32,
- *     and the sums are scaled back exactly (unless the result is an fp32
- *     subnormal); the scale comes from the largest finite magnitude (Inf and
- *     NaN entries stay Inf and NaN), a row or column with no finite nonzero
- *     value keeps scale 1, one whose largest is below 2^-112 takes 2^127.
+ *     bits; each operand row or column along which the sum runs is scaled by a
+ *     power of two that brings its largest magnitude into [2^11, 2^15), so its
+ *     values are fp16 values (exactly, unless 2^25 or more below that largest
+ *     one: then within 2^-36 of it), the products are exact in fp32, and the
+ *     sums are scaled back exactly (unless the result is an fp32 subnormal);
+ *     the scale comes from the largest finite magnitude (Inf and NaN entries
+ *     stay Inf and NaN), a row or column with no finite nonzero value keeps
+ *     scale 1 (dgrad: one whose largest is below 2^-112 takes 2^127).
  *   dgrad: grad_input [M, N] = tf32(grad_output [M, K]) @ tf32(weight [K, N]):
  *     grad_output scaled per row, weight per column, the scales undone in the
  *     GEMM's epilogue.
  *   wgrad: grad_weight [N, K] = tf32(grad_output [M, N])^T @ tf32(inp [M, K]):
- *     both scaled per column, undone where the reduction planes are added.
+ *     both scaled per column; inp's scales are found as its rows stream by, and
+ *     the sums so far follow a scale that changes.
  * Limits: the column counts (K and N) % 8 == 0; dgrad 3K, N < 2^22 and
  *   3K*N < 2^30; wgrad M*N, M*K, N*K < 2^30; 16-byte aligned tensors.
  * Workspace: the *_workspace_size bytes, 256-byte aligned (dgrad: the fp16
  *   copies, M K + K N values, the row and column exponents and the
- *   column-max slabs; wgrad: the fp16 copies, M N + M K values, the column
- *   exponents, column-max slabs and the fp32 planes of the reduction chunks,
- *   at least one). */
+ *   column-max slabs; wgrad: the transposed fp16 copy of grad_output, its
+ *   columns' exponents and column-max slabs, and the fp32 planes of the
+ *   reduction chunks where there are several; at least the size of an fp16
+ *   copy of both operands with their exponents, slabs and planes). */
 size_t moe_router_dgrad_tf32_workspace_size(int64_t M, int64_t K, int64_t N);
 int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const float *weight, int64_t N,
                           float *grad_input, void *workspace, size_t workspace_bytes, void *stream);

@@ -161,3 +161,32 @@ def test_router_tf32_inf_and_nan_entries(pkg, dev, which):
     assert int((~fin).sum()) > 0 and int(fin.sum()) > 0
     err = (got[fin].double() - ref[fin].double()).abs()
     assert bool((err <= 1e-4 * absprod[fin].double() + 1e-5).all())
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 8),          # one reduction row
+    (63, 64, 264),      # less than a stage, one column past a column tile
+    (193, 72, 256),     # four stages: the ring's slots wrap; 5 row blocks of the 8
+    (700, 256, 1000),   # chunks of the reduction, the last one shorter
+    (2049, 320, 72),    # a chunk of one row
+    (300, 648, 512),    # three row tiles
+])
+def test_router_wgrad_tf32_edges_and_growing_columns(pkg, dev, M, N, K):
+    # Columns of inp whose magnitudes grow along the rows (the scale found first does not hold), a column that is zero
+    # until the last row, a value that tf32 rounds to Inf's neighbour, and zero columns; the reference is the float64
+    # sum of the tf32-rounded operands' products, at the bound of this file.
+    g = torch.Generator().manual_seed(M + 3 * N + K)
+    go = torch.randn(M, N, generator=g)
+    x = torch.randn(M, K, generator=g)
+    x[:, 1] *= 10.0 ** torch.linspace(-20, 18, M)
+    x[:, 2] = 0.0
+    x[M - 1, 2] = 1e-12
+    x[:, 3] = 0.0
+    x[:, 5] *= 10.0 ** torch.linspace(12, -25, M)
+    x[M // 2, 6] = 3.4e38
+    go[M // 2] *= 1e-3  # keeps column 6 finite
+    got = pkg.ops.router_wgrad_tf32(go.to(dev), x.to(dev)).cpu().double()
+    a, b = ref_torch.round_tf32_rne(go).double(), ref_torch.round_tf32_rne(x).double()
+    ref = a.t() @ b
+    excess = (got - ref).abs() - (1e-4 * (a.abs().t() @ b.abs()) + 2.0 ** -126)
+    assert bool(torch.isfinite(got).all())
+    assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
