@@ -36,6 +36,7 @@ SOURCES = [
     "expert_stream.hip",
     "grouped_gemm_bwd.hip",
     "router.hip",
+    "router_dgrad.hip",
     "router_wgrad.hip",
     "cast.hip",
 ]

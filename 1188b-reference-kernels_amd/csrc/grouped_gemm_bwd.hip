@@ -2134,8 +2134,8 @@ bool dgrad_pp_tails(int64_t M, int64_t N, int64_t G) {
          N >= std::max<int64_t>(3 * kBK, gemm::kTailsMinK);
 }
 
-// tf32 router dgrad, grad_input [M, N] = grad_output [M, K] weight [K, N]. With more than 160 rows and a
-// reduction of whole steps (K % 64 == 0, K >= 192) it runs on the fp16 matrix cores: grad_output's rows and
+// tf32 router dgrad, grad_input [M, N] = grad_output [M, K] weight [K, N]. Reductions of at most 320 run the
+// weight-stationary kernel of router_dgrad.hip; longer ones run here on the fp16 matrix cores: grad_output's rows and
 // weight's columns are scaled by powers of two into the fp16 range (one exact fp16 product per tf32
 // product) and the GEMM's epilogue undoes both scales; otherwise it runs on the bf16 hi/lo split (three
 // products, a 3K reduction). Workspace (byte offsets, each 256-byte aligned): fp16 path: the fp16 copies
@@ -2151,6 +2151,10 @@ DgradTf32Layout dgrad_tf32_layout(int64_t M, int64_t K, int64_t N) {
   using moe::align_up;
   DgradTf32Layout l{};
   l.f16 = MOE_ROUTER_DGRAD_F16 != 0;
+  if (l.f16 && moe::router_dgrad_applies(K)) {
+    l.total = moe::router_dgrad_layout(M, K, N).total;
+    return l;
+  }
   if (!l.f16) {
     l.total = align_up(static_cast<size_t>(M) * 3 * K * 2) + align_up(static_cast<size_t>(3 * K) * N * 2);
     return l;
@@ -2374,6 +2378,10 @@ int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const 
                 workspace == nullptr ? size_t(0) : workspace_bytes);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (l.f16 && router_dgrad_applies(K)) {
+    launch_router_dgrad(grad_output, M, K, weight, N, grad_input, workspace, s);
+    return check_launch(fn);
+  }
   if (l.f16) {
     char *w = static_cast<char *>(workspace);
     uint16_t *a16 = reinterpret_cast<uint16_t *>(w + l.a16);

@@ -1,0 +1,296 @@
+// tf32 router input gradient: grad_input [M, N] = tf32(grad_output [M, K]) tf32(weight [K, N]), fp32 in and out, on the
+// fp16 matrix cores (tf32_device.h), for reductions of at most 320 (the number of experts).
+//
+// The work is the output: 4 M N bytes written (537 MB at 16384 x 8192) for a reduction of a few hundred, so the kernel
+// is built around the stores:
+//   * the weight stays where it is used: a wavefront owns 64 columns and holds all their MFMA fragments (40 of 16 bytes
+//     a lane at K = 320) in registers for its whole run; only grad_output's rows stream by, through a ring of three LDS
+//     stages of 64 rows that the 8 wavefronts (512 columns) share, with one barrier a stage;
+//   * block j of a wavefront's four is columns 4 c + j, c = 0 .. 15, so a lane's four accumulators of a row are four
+//     neighbouring columns: one 16-byte store, 256 contiguous bytes of a row over 16 lanes;
+//   * nothing waits for the stores: they are older than the loads that the next stages wait for only by whole stages.
+// grad_output is scaled per row, weight per column (transposed, so that both are read along the reduction), in one launch
+// before; the epilogue undoes both.
+// Measured (MI355X, us for the call): 16384 x 320 x 8192 232 -> 138 (the GEMM 209 -> 107-117: 4.6-5.0 TB/s of output;
+// its operands' preparation 25 in four launches -> 18 in one), 16384 x 64 x 7168 164 -> 98, 100 x 64 x 7168 24 -> 17.
+// Before: 128 x 128 tiles of five reduction steps, 32 bytes of a row per store, still what longer reductions run
+// (grouped_gemm_dgrad128_kernel in grouped_gemm_bwd.hip).
+#include <algorithm>
+#include <type_traits>
+
+#include "gemm_device.h"
+#include "tf32_device.h"
+
+namespace moe {
+namespace {
+
+using namespace gemm;
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+
+constexpr int kRowsStage = 64, kColsWave = 64, kColsTile = 512;
+
+struct DgradArgs {
+  const uint16_t *a;    // [M64, 64 kKS2] fp16: scaled rows of grad_output, zeros past K and M
+  const uint16_t *b;    // [N, 64 kKS2] fp16: scaled columns of weight
+  const int32_t *a_exp; // [M64]
+  const int32_t *b_exp; // [N]
+  float *out;
+  int64_t M, N;
+  int64_t chunk;        // rows of a unit (a multiple of 64)
+  int col_tiles, units;
+};
+
+// kKS2: 64-deep steps of the reduction.
+template <int kKS2>
+__global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
+  constexpr int kKS = 2 * kKS2;                  // MFMAs per block
+  constexpr int kRowB = 128 * kKS2;              // bytes of a row
+  constexpr int kStage = kRowsStage * kRowB;     // 8 kKS2 KiB
+  constexpr int kExp = kRowsStage * 4;           // the rows' exponents
+  constexpr int kSlots = 3;
+  constexpr int kDma = kKS2;                     // 1 KiB blocks per wavefront and stage
+  constexpr int kStores = kRowsStage / 16 * 4;   // per lane and stage
+  constexpr int kLds = kSlots * (kStage + kExp);
+  static_assert(kLds <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(1024))) char smem[kLds];
+  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char *)smem));
+  const uint32_t lds_exp = lds + kSlots * kStage;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int c16 = lane & 15, q = lane >> 4;
+  const int b = static_cast<int>(blockIdx.x), P = static_cast<int>(gridDim.x);
+  const int u = (b % 8) * (P / 8) + b / 8;  // an XCD takes neighbouring units: the column tiles of one chunk of rows
+  if (u >= p.units) return;
+  const int ct = u % p.col_tiles;
+  const int64_t m0 = static_cast<int64_t>(u / p.col_tiles) * p.chunk, m1 = min(p.M, m0 + p.chunk);
+  const int stages = static_cast<int>((m1 - m0 + kRowsStage - 1) / kRowsStage);
+
+  // ---- rows: block wave + 8 j of a stage; 16-byte chunks of a row are XORed with the row within each 128 bytes. The
+  // offsets are formed anew for each stage (from a lane index the compiler takes for another): the registers are the
+  // weight's.
+  auto dma = [&](int st) {
+    const int sc = min(st, stages - 1);  // past the last stage the last one again, into a slot nothing reads any more
+    const int64_t m = m0 + static_cast<int64_t>(sc) * kRowsStage;
+    const int slot = st % kSlots;
+    if (wave == 0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.a_exp + m, kExp), (lds_void *)(uintptr_t)(lds_exp + slot * kExp), 4, lane * 4, 0, 0, 0);
+#endif
+    }
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a + m * (kRowB / 2), kStage);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+#pragma unroll
+    for (int j = 0; j < kDma; ++j) {
+      const int at = (wave + 8 * j) * 64 + ln;  // chunk of the stage, as it lies in LDS
+      const int r = at / (8 * kKS2), c = at % (8 * kKS2);
+      dma16b(ra, (lds_void *)(uintptr_t)(lds + slot * kStage + (wave + 8 * j) * 1024), r * kRowB + ((c & ~7) | ((c ^ r) & 7)) * 16, 0);
+    }
+  };
+  dma(0);
+  dma(1);
+
+  // ---- this wavefront's columns
+  const int64_t n0 = static_cast<int64_t>(ct) * kColsTile + wave * kColsWave + 4 * c16;
+  const bool in = n0 < p.N;  // N % 8 == 0: a lane's four columns are all valid or all past N
+  f16x8 fb[kKS][4];
+  int eb[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t n = in ? n0 + j : 0;
+    eb[j] = p.b_exp[n];
+#pragma unroll
+    for (int ks = 0; ks < kKS; ++ks) fb[ks][j] = *reinterpret_cast<const f16x8 *>(p.b + n * (kRowB / 2) + ks * 32 + q * 8);
+  }
+  const uint32_t ld = static_cast<uint32_t>(p.N) * 4u;
+  const uint32_t o_lane = in ? static_cast<uint32_t>(4 * q) * ld + static_cast<uint32_t>(n0) * 4u : kNoAccess;
+  const uint32_t a_lane = static_cast<uint32_t>(c16) * kRowB + (((q ^ c16) & 7) << 4);
+
+  for (int st = 0; st < stages; ++st) {
+    // The stage's DMA has landed: after it came the stores of two stages and the next stage's DMA.
+    if (st == 0) wait_dma();
+    else wait_vm_n<2 * kStores + kDma>();
+    barrier();
+    dma(st + 2);  // into the slot of stage st - 1, which every wavefront has left
+    const int64_t m = m0 + static_cast<int64_t>(st) * kRowsStage;
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + m * p.N, static_cast<uint32_t>(min<int64_t>(m1 - m, kRowsStage)) * ld);
+    const uint32_t base = lds + (st % kSlots) * kStage + a_lane, ebase = lds_exp + (st % kSlots) * kExp;
+#pragma unroll 1
+    for (int i = 0; i < kRowsStage / 16; ++i) {
+      f32x4 acc[4];
+      f16x8 fa[2];
+      // chunk 4 ks + q of the row: its 128 bytes, and within them the swizzled place (the odd ks's differs by 64 bytes)
+      auto read = [&](int ks) {
+        return *reinterpret_cast<const lds_f16x8 *>((uintptr_t)((base ^ ((ks & 1) << 6)) + i * 16 * kRowB + (ks >> 1) * 128));
+      };
+      fa[0] = read(0);
+      const i32x4 ea = *reinterpret_cast<const lds_i32x4 *>((uintptr_t)(ebase + (i * 16 + 4 * q) * 4));
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        if (ks + 1 < kKS) fa[(ks + 1) & 1] = read(ks + 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[ks & 1], fb[ks][j], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);  // no further reads ahead: the registers are the weight's
+      }
+      // acc[j] register t: row 16 i + 4 q + t, column n0 + j
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        u32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(__builtin_ldexpf(acc[j][t], -(ea[t] + eb[j])));
+#if defined(__HIP_DEVICE_COMPILE__)
+        __builtin_amdgcn_raw_buffer_store_b128(v, ro, static_cast<int>(in ? o_lane + static_cast<uint32_t>(i * 16 + t) * ld : kNoAccess), 0, 0);
+#else
+        (void)ro;
+        (void)o_lane;
+        (void)v;
+#endif
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  wait_dma();  // no LDS DMA outlives the workgroup
+}
+
+// Both operands in one launch. Blocks [0, wb): 64 columns of weight [K, N] each, all K <= 64 kV / 4 rows: its columns'
+// largest finite magnitudes, their exponents, the scaled columns as rows of b (kp long, zeros past K). The other blocks:
+// four rows of grad_output each, one per wavefront (rows past M: zeros and exponent 0).
+template <int kV>
+__global__ __launch_bounds__(256) void router_dgrad_prepare_kernel(const float *w, const float *go, int64_t M, int64_t M64, int K, int64_t N,
+                                                                   int kp, int wb, uint16_t *a, uint16_t *bt, int32_t *a_exp, int32_t *b_exp) {
+  constexpr int kRows = 16 * kV;              // rows of weight held by a block
+  constexpr int kPitch = kRows + 8;           // LDS row of a column, in values (16-byte rows; a bank offset per column)
+  __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kPitch];
+  __shared__ float red[16][64];
+  const int t = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) < wb) {
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 64;
+    const int c = (t & 15) * 4, r0 = t >> 4;
+    u32x4 v[kV];
+    float mx[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kV; ++i) {
+      const int r = r0 + 16 * i;
+      v[i] = r < K && n0 + c < N ? *reinterpret_cast<const u32x4 *>(w + static_cast<int64_t>(r) * N + n0 + c) : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int i = 0; i < kV; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) mx[k] = fmaxf(mx[k], finite_abs(__uint_as_float(v[i][k])));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) red[r0][c + k] = mx[k];
+    __syncthreads();
+    int e[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) m = fmaxf(m, red[i][c + k]);
+      e[k] = scale_exp(m);
+      if (r0 == 0 && n0 + c + k < N) b_exp[n0 + c + k] = e[k];
+    }
+#pragma unroll
+    for (int i = 0; i < kV; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        tile[(c + k) * kPitch + r0 + 16 * i] =
+            __builtin_bit_cast(uint16_t, static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(v[i][k])), e[k])));
+    __syncthreads();
+    const int per = kp / 8;  // 16-byte pieces of a column
+    for (int i = t; i < 64 * per; i += 256) {
+      const int n = i / per, k = i - n * per;
+      if (n0 + n < N) *reinterpret_cast<u32x4 *>(bt + (n0 + n) * kp + k * 8) = *reinterpret_cast<const u32x4 *>(&tile[n * kPitch + k * 8]);
+    }
+    return;
+  }
+  const int64_t m = static_cast<int64_t>(blockIdx.x - wb) * 4 + t / kWave;
+  const int lane = t % kWave;
+  if (m >= M64) return;
+  constexpr int kU = (kRows + 255) / 256;  // 4 values a lane at a time
+  u32x4 v[kU];
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < kU; ++i) {
+    const int k = (lane + i * kWave) * 4;
+    v[i] = m < M && k < K ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(go + m * K + k)) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mx = fmaxf(mx, finite_abs(__uint_as_float(v[i][j])));
+  }
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+  const int e = scale_exp(mx);
+  if (lane == 0) a_exp[m] = e;
+#pragma unroll
+  for (int i = 0; i < kU; ++i) {
+    const int k = (lane + i * kWave) * 4;
+    if (k >= kp) continue;
+    uint32_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      h[j] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(v[i][j])), e)));
+    *reinterpret_cast<u32x2 *>(a + m * kp + k) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+  }
+}
+
+int64_t round64(int64_t v) { return ceil_div(v, 64) * 64; }
+
+}  // namespace
+
+bool router_dgrad_applies(int64_t K) { return K > 0 && K <= 320; }
+
+RouterDgradLayout router_dgrad_layout(int64_t M, int64_t K, int64_t N) {
+  RouterDgradLayout l;
+  const int64_t kp = round64(K), M64 = round64(M);
+  auto take = [&](int64_t bytes) {
+    const size_t at = l.total;
+    l.total += static_cast<size_t>(ceil_div(bytes, 256) * 256);
+    return at;
+  };
+  l.a = take(M64 * kp * 2);
+  l.b = take(N * kp * 2);
+  l.a_exp = take(M64 * 4);
+  l.b_exp = take(N * 4);
+  return l;
+}
+
+void launch_router_dgrad(const float *go, int64_t M, int64_t K, const float *w, int64_t N, float *out, void *workspace, hipStream_t s) {
+  const RouterDgradLayout l = router_dgrad_layout(M, K, N);
+  char *ws = static_cast<char *>(workspace);
+  const int64_t kp = round64(K), M64 = round64(M), wb = ceil_div(N, 64);
+  uint16_t *a = reinterpret_cast<uint16_t *>(ws + l.a), *b = reinterpret_cast<uint16_t *>(ws + l.b);
+  int32_t *a_exp = reinterpret_cast<int32_t *>(ws + l.a_exp), *b_exp = reinterpret_cast<int32_t *>(ws + l.b_exp);
+  DgradArgs p;
+  p.a = a;
+  p.b = b;
+  p.a_exp = a_exp;
+  p.b_exp = b_exp;
+  p.out = out;
+  p.M = M;
+  p.N = N;
+  p.col_tiles = static_cast<int>(ceil_div(N, kColsTile));
+  // A unit for every CU, of whole stages.
+  p.chunk = round64(std::max<int64_t>(64, ceil_div(M, std::max<int64_t>(1, num_cus() / p.col_tiles))));
+  p.units = static_cast<int>(ceil_div(M, p.chunk)) * p.col_tiles;
+  const dim3 grid(static_cast<uint32_t>((p.units + 7) / 8 * 8)), block(512), pgrid(static_cast<uint32_t>(wb + M64 / 4));
+  auto go_ = [&](auto steps) {
+    constexpr int kSteps = decltype(steps)::value;
+    router_dgrad_prepare_kernel<4 * kSteps><<<pgrid, dim3(256), 0, s>>>(w, go, M, M64, static_cast<int>(K), N, static_cast<int>(kp),
+                                                                        static_cast<int>(wb), a, b, a_exp, b_exp);
+    router_dgrad_kernel<kSteps><<<grid, block, 0, s>>>(p);
+  };
+  switch (kp / 64) {
+    case 1: go_(std::integral_constant<int, 1>{}); break;
+    case 2: go_(std::integral_constant<int, 2>{}); break;
+    case 3: go_(std::integral_constant<int, 3>{}); break;
+    case 4: go_(std::integral_constant<int, 4>{}); break;
+    default: go_(std::integral_constant<int, 5>{}); break;
+  }
+}
+
+}  // namespace moe

@@ -46,4 +46,13 @@ void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, co
 void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const int32_t *exp, const float *inp, int64_t M, int64_t N,
                          int64_t K, float *planes, float *out, hipStream_t s);
 
+// ---- router dgrad (router_dgrad.hip): reductions of at most 320
+
+bool router_dgrad_applies(int64_t K);
+struct RouterDgradLayout {  // workspace, byte offsets
+  size_t a = 0, b = 0, a_exp = 0, b_exp = 0, total = 0;
+};
+RouterDgradLayout router_dgrad_layout(int64_t M, int64_t K, int64_t N);
+void launch_router_dgrad(const float *go, int64_t M, int64_t K, const float *w, int64_t N, float *out, void *workspace, hipStream_t s);
+
 }  // namespace moe

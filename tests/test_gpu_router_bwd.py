@@ -190,3 +190,28 @@ def test_router_wgrad_tf32_edges_and_growing_columns(pkg, dev, M, N, K):
     excess = (got - ref).abs() - (1e-4 * (a.abs().t() @ b.abs()) + 2.0 ** -126)
     assert bool(torch.isfinite(got).all())
     assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, 8),         # one row, one lane's columns
+    (65, 256, 520),     # a stage and a row; a column past a column tile
+    (4100, 128, 1032),  # chunks of several stages: the ring's slots wrap
+    (12345, 192, 2056), # five column tiles, uneven chunks
+    (70, 320, 64),      # the longest reduction of the weight-stationary kernel
+    (70, 328, 64),      # and one past it (128-row tiles)
+])
+def test_router_dgrad_tf32_edges(pkg, dev, M, K, N):
+    # Against the float64 sum of the tf32-rounded operands' products, at the bound of this file; guard rows around
+    # the output stay as they are.
+    g = torch.Generator(device=dev).manual_seed(M + 3 * K + N)
+    go = torch.randn(M, K, generator=g, device=dev) * 10.0 ** torch.linspace(-20, 10, M, device=dev)[:, None]
+    w = torch.randn(K, N, generator=g, device=dev) * 10.0 ** torch.linspace(-8, 8, N, device=dev)
+    nbytes = pkg._lib.lib().moe_router_dgrad_tf32_workspace_size(M, K, N)
+    ws = torch.full((nbytes,), 0xAB, dtype=torch.uint8, device=dev)
+    buf = torch.full((M + 2, N), 3.0, device=dev)
+    pkg._lib.call("moe_router_dgrad_tf32", pkg._lib.ptr(go), M, K, pkg._lib.ptr(w), N, pkg._lib.ptr(buf[1:]), pkg._lib.ptr(ws), nbytes,
+                  pkg._lib.stream_handle())
+    a, b = ref_torch.round_tf32_rne(go.cpu()).double(), ref_torch.round_tf32_rne(w.cpu()).double()
+    excess = (buf[1:M + 1].cpu().double() - a @ b).abs() - (1e-4 * (a.abs() @ b.abs()) + 2.0 ** -126)
+    assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
+    assert bool((buf[0] == 3.0).all()) and bool((buf[M + 1] == 3.0).all()), "stored outside grad_input"
