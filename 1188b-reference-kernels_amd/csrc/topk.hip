@@ -1,5 +1,7 @@
 // Router top-k (+ routing mask and merge probs), one wavefront per row; the
 // per-row routine and its math citation are in topk_device.h.
+#include <type_traits>
+
 #include "topk_device.h"
 
 namespace moe {
@@ -16,6 +18,22 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(const float *logits, int
   if (t >= T) return;
   const float *row = logits + t * E;
   topk_row<kEPL>([&](int e) { return row[e]; }, t, E, k, values, indices, routing_map, probs);
+}
+
+// go(n) with the slots per lane that E experts need (n = 64-element pieces, 16 above 512 experts).
+template <typename Go>
+void by_slots(int E, Go go) {
+  switch ((E + kWave - 1) / kWave) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    default: go(std::integral_constant<int, 16>{}); break;
+  }
 }
 
 }  // namespace
@@ -38,11 +56,10 @@ int moe_topk(const float *logits, int64_t T, int64_t E, int64_t k, float *values
   if (grid > 0x7fffffff) return fail(MOE_ERR_CAPACITY, "moe_topk: T=%lld too large", (long long)T);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int e = static_cast<int>(E), kk = static_cast<int>(k);
-  if (E <= 64) topk_kernel<1><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
-  else if (E <= 128) topk_kernel<2><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
-  else if (E <= 256) topk_kernel<4><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
-  else if (E <= 512) topk_kernel<8><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
-  else topk_kernel<16><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
+  auto go = [&](auto epl) {
+    topk_kernel<decltype(epl)::value><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
+  };
+  by_slots(e, go);
   return check_launch("moe_topk");
 }
 

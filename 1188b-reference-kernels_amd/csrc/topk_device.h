@@ -8,13 +8,19 @@
 // zeros(T,E,bool).scatter_(1, idx, True) (case18...py:86-88) and the merge
 // probs are softmax over the k selected values (fp32), scattered to [T, E].
 //
-// Lane l holds elements l, l+64, ... (kEPL per lane) as 32-bit order keys.
-// Each of the k rounds takes the wave-wide maximum key over the lanes' current
-// bests (DPP row operations, no LDS crossbar), then the smallest index holding
-// it (a ballot when a lane holds one element, else a DPP minimum), so ties go
-// to the smaller index; the owning lane retires that element and refreshes its
-// own best.  Lane j keeps round j's winner, so lanes < k store values/indices
-// coalesced.
+// Lane l holds elements l, l+64, ... (kEPL per lane) as 32-bit order keys,
+// sorted once (odd-even transposition: only neighbours trade places, so equal
+// keys stay in slot order; up to 8 elements). Each of the k rounds takes the wave-wide maximum of
+// the lanes' first keys (DPP row operations, no LDS crossbar); a ballot names
+// the lane that holds it, whose list moves up by one. Where several lanes hold
+// it, the smallest index among their first slots wins (a DPP minimum), so ties
+// go to the smaller index. Lane j keeps round j's winner, so lanes < k store
+// values/indices coalesced.
+// What bounds it is the chain of a round, not the bytes; 16384 rows, k = 8, us, with
+// the index always found by a second DPP chain and the winner's list searched
+// again every round, and with this form: 320 experts 29.5 and 19.3 (8 slots a lane
+// before, 5 now), 160 21.6 and 14.4, 64 10.6 and 9.7. Above 8 slots the sort costs
+// more than the searches (1024 experts: 58 against 50), so the list stays unsorted.
 #pragma once
 
 #include "moe_common.h"
@@ -76,70 +82,87 @@ __device__ __forceinline__ void topk_row(Load load, int64_t t, int E, int k, flo
                                          uint8_t *routing_map, float *probs) {
   const int lane = lane_id();
   float val[kEPL];
-  uint32_t key[kEPL];
-  uint32_t live = 0;  // bit s: element lane + 64 s not yet selected
+  constexpr bool kSorted = kEPL <= 8;
+  uint32_t key[kEPL], slot[kEPL];  // key 0 = nothing left (every float's order key is above 0)
 #pragma unroll
   for (int s = 0; s < kEPL; ++s) {
     const int e = s * kWave + lane;
     val[s] = 0.0f;
     key[s] = 0u;
+    slot[s] = s;
     if (e < E) {
       val[s] = load(e);
       key[s] = order_key(val[s]);
-      live |= 1u << s;
     }
   }
-  const uint32_t present = live;
-
-  // Best of this lane: largest live key, the smaller slot on equal keys; key
-  // 0 = nothing left (every float's order key is above 0).
-  uint32_t best_key = 0, best_slot = 0;
-  auto lane_best = [&]() {
-    best_key = 0;
-    best_slot = 0;
+  if constexpr (kSorted) {
 #pragma unroll
-    for (int s = 0; s < kEPL; ++s) {
-      if ((live & (1u << s)) && key[s] > best_key) {
-        best_key = key[s];
-        best_slot = s;
+    for (int r = 0; r < kEPL; ++r) {
+#pragma unroll
+      for (int s = r % 2; s + 1 < kEPL; s += 2) {
+        const bool up = key[s + 1] > key[s];
+        const uint32_t ka = key[s], kb = key[s + 1], sa = slot[s], sb = slot[s + 1];
+        key[s] = up ? kb : ka;
+        key[s + 1] = up ? ka : kb;
+        slot[s] = up ? sb : sa;
+        slot[s + 1] = up ? sa : sb;
+      }
+    }
+  }
+  // The lane's first: its largest key, the smaller slot on equal keys.
+  uint32_t first_key, first_slot;
+  auto first = [&]() {
+    first_key = key[0];
+    first_slot = slot[0];
+    if constexpr (!kSorted) {
+#pragma unroll
+      for (int s = 1; s < kEPL; ++s) {
+        const bool up = key[s] > first_key;
+        first_key = up ? key[s] : first_key;
+        first_slot = up ? s : first_slot;
       }
     }
   };
+  first();
 
-  lane_best();
-  float my_val = 0.0f;
+  uint32_t chosen = 0;  // bit s: element lane + 64 s selected
   int my_idx = 0;
   for (int j = 0; j < k; ++j) {
-    const uint32_t kmax = wave_reduce_u32<true>(best_key);
-    int widx;
-    if constexpr (kEPL == 1) {
-      widx = __builtin_ctzll(__ballot(best_key == kmax));  // element index = lane
+    const uint32_t kmax = wave_reduce_u32<true>(first_key);
+    const uint64_t holders = __ballot(first_key == kmax);
+    int widx, wlane = __builtin_ctzll(holders);
+    if (kEPL == 1) {
+      widx = wlane;
+    } else if ((holders & (holders - 1)) == 0) {
+      widx = __builtin_amdgcn_readlane(static_cast<int>(first_slot), wlane) * kWave + wlane;
     } else {
-      const uint32_t cand = best_key == kmax ? best_slot * kWave + lane : 0xffffffffu;
-      widx = static_cast<int>(wave_reduce_u32<false>(cand));
+      widx = static_cast<int>(wave_reduce_u32<false>(first_key == kmax ? first_slot * kWave + lane : 0xffffffffu));
+      wlane = widx % kWave;
     }
-    const int wlane = widx % kWave, wslot = widx / kWave;
-    float wval = 0.0f;
     if (lane == wlane) {
+      chosen |= 1u << first_slot;
+      if constexpr (kSorted) {
 #pragma unroll
-      for (int s = 0; s < kEPL; ++s)
-        if (s == wslot) wval = val[s];
-      live &= ~(1u << wslot);
-      lane_best();
+        for (int s = 0; s + 1 < kEPL; ++s) {
+          key[s] = key[s + 1];
+          slot[s] = slot[s + 1];
+        }
+        key[kEPL - 1] = 0u;
+      } else {
+#pragma unroll
+        for (int s = 0; s < kEPL; ++s) key[s] = s == static_cast<int>(first_slot) ? 0u : key[s];
+      }
+      first();
     }
-    wval = readlane_f32(wval, wlane);
-    if (lane == j) {
-      my_val = wval;
-      my_idx = widx;
-    }
+    if (lane == j) my_idx = widx;
   }
+  const float my_val = lane < k ? load(my_idx) : 0.0f;  // (the key does not hold -0 or a NaN's bits)
   if (lane < k) {
     values[t * k + lane] = my_val;
     indices[t * k + lane] = my_idx;
   }
 
   if (routing_map != nullptr || probs != nullptr) {
-    const uint32_t chosen = present & ~live;
     float inv_sum = 0.0f, vmax = 0.0f;
     if (probs != nullptr) {
       vmax = readlane_f32(my_val, 0);

@@ -1,0 +1,45 @@
+"""GPU: the top-k's slot lists and the row-id map's one-launch form, at the sizes where they can go wrong; whole numbers
+and copies, so equal bit for bit to the oracle."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import ref_torch
+from conftest import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("E", [1, 60, 64, 65, 128, 129, 192, 193, 257, 320, 321, 384, 448, 449, 512, 513, 1024])
+@pytest.mark.parametrize("levels", [2, 7, 0])
+def test_topk_slots_and_ties(pkg, dev, E, levels):
+    # Few distinct values: ties inside a lane's list, between lanes, and between both; signed zeros, infinities, NaN.
+    g = torch.Generator().manual_seed(E + levels)
+    T, k = 37, min(E, 64)
+    x = torch.randint(0, levels, (T, E), generator=g).float() - levels // 2 if levels else torch.randn(T, E, generator=g)
+    special = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), 3.4e38])
+    hit = torch.rand(T, E, generator=g) < 0.1
+    x[hit] = special[torch.randint(0, 6, (int(hit.sum()),), generator=g)]
+    for kk in {1, min(E, 8), k}:
+        values, indices, mask = pkg.ops.topk(x.to(dev), kk, with_mask=True)
+        rv, ri = ref_torch.topk(x, kk)
+        assert torch.equal(indices.cpu(), ri), f"E={E} k={kk}"
+        assert_bits_equal(values, rv, f"E={E} k={kk}")
+        assert torch.equal(mask.cpu(), torch.zeros(T, E, dtype=torch.bool).scatter_(1, ri, True))
+
+
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 255, 256, 257])
+@pytest.mark.parametrize("E", [1, 31, 32, 33, 60, 64, 80, 256, 272, 1024])
+def test_row_id_map_one_launch_sizes(pkg, dev, T, E):
+    # T <= 256 and a mask of at most 64 KiB (16 KiB without 16-byte loads) is one launch; the sizes lie on both sides.
+    g = torch.Generator().manual_seed(T * 1000 + E)
+    for rm in (torch.rand(T, E, generator=g) < 0.15, torch.ones(T, E, dtype=torch.bool), torch.zeros(T, E, dtype=torch.bool)):
+        R = int(rm.sum())
+        row_em, row_tm = ref_torch.row_id_map(rm)
+        m = rm.to(torch.uint8) * torch.randint(1, 256, (T, E), generator=g).to(torch.uint8)  # any nonzero byte selects
+        got = pkg.ops.row_id_map(m.to(dev), expert_major_i32=True, expert_offsets=True, src_rows=R)
+        assert torch.equal(got["expert_major"].cpu(), row_em) and torch.equal(got["token_major"].cpu(), row_tm)
+        assert torch.equal(got["expert_major_i32"].cpu().long(), row_em)
+        assert torch.equal(got["expert_offsets"].cpu(), ref_torch.expert_offsets(rm))
+        assert torch.equal(got["src_token"].cpu().long(), rm.t().nonzero()[:, 1])
