@@ -150,6 +150,14 @@ def ptr(t) -> int | None:
     return t.data_ptr() if t.numel() > 0 else None
 
 
+# torch.cuda.current_stream() builds a Stream object on every call (2.7 us of host time, a sixth of a small op's); the raw
+# handle of the same stream takes 0.1 us.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream_handle() -> int:
     """hipStream_t of torch's current stream on the current device."""
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
