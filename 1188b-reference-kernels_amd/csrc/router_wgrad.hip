@@ -15,9 +15,9 @@
 //     LDS stages of 64 reduction rows, shared by the 8 wavefronts (256 columns);
 //   * M is cut into chunks so that there is a unit for every CU; the units of one XCD share a chunk, whose part of the
 //     small operand then stays in its L2. The planes of the chunks are added in order.
-// Measured (MI355X, 16384 x 320 x 8192, us): 395 -> 175 for the whole call; the GEMM 124-134 (4.0-4.3 TB/s of inp), the
+// Measured (MI355X, 16384 x 320 x 8192, us): 395 -> 171 for the whole call; the GEMM 120-134 (4.0-4.5 TB/s of inp; 150 without the multiplications and conversions, so it is the loads), the
 // planes' sum 16, grad_output's maxima and copy 17. Before: column maxima of inp 90, its fp16 copy 180, a GEMM on the
-// copies 143, the sum 10. 16384 x 64 x 7168: 307 -> 136; 4096 x 128 x 7168: 98 -> 74; 100 x 64 x 7168: 39 -> 19.
+// copies 143, the sum 10. 16384 x 64 x 7168: 307 -> 101; 4096 x 128 x 7168: 98 -> 49; 100 x 64 x 7168: 39 -> 19.
 #include <algorithm>
 #include <type_traits>
 
@@ -51,8 +51,8 @@ struct WgradArgs {
   int col_tiles, row_tiles, units;
 };
 
-// kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets).
-template <int kMI, bool kWide>
+// kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets). kNt: non-temporal loads of it.
+template <int kMI, bool kWide, bool kNt>
 __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
   constexpr int kStage = kMI * 16 * kRowB;
   constexpr int kSlots = 3;
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     // The rows' offsets are in the vector offset: the scalar one is not part of the range check.
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) dst[r] = __builtin_amdgcn_raw_buffer_load_b64(rb, static_cast<int>(b_off + (row + r) * ldb), 0, 2);
+    for (uint32_t r = 0; r < 8; ++r) dst[r] = __builtin_amdgcn_raw_buffer_load_b64(rb, static_cast<int>(b_off + (row + r) * ldb), 0, kNt ? 2 : 0);
 #else
     (void)row;
     (void)b_off;
@@ -300,8 +300,9 @@ RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K) {
   pl.mi = K >= kWideK || blocks <= 4 ? 4 : blocks <= 8 ? 8 : blocks <= 16 ? 16 : 20;
   pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 16 * pl.mi));
   const int64_t tiles = pl.row_tiles * std::max<int64_t>(1, ceil_div(K, kColsTile));
-  // A unit for every CU, of at least 128 rows; and a chunk of inp below 2 GiB (32-bit offsets).
-  int64_t s = std::min(ceil_div(256, tiles), std::max<int64_t>(1, M / 128));
+  // At most a unit for every CU (a second round for a few more costs a whole one: 16384 x 64 x 7168, 28 tiles, 10 chunks
+  // 139 us, 9 101), of at least 128 rows; and a chunk of inp below 2 GiB (32-bit offsets).
+  int64_t s = std::max<int64_t>(1, std::min(256 / tiles, M / 128));
   if (K < kWideK) s = std::max(s, ceil_div(M * K, (int64_t(1) << 29) - 64 * K));
   pl.c = std::max<int64_t>(1, ceil_div(ceil_div(M, s), kBK)) * kBK;
   pl.s = std::max<int64_t>(1, ceil_div(M, pl.c));
@@ -332,16 +333,20 @@ void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const 
   const int64_t units = pl.s * p.col_tiles * pl.row_tiles;
   p.units = static_cast<int>(units);
   const dim3 grid(static_cast<uint32_t>((units + 7) / 8 * 8)), block(512);
-  if (K >= kWideK) {
-    router_wgrad_kernel<4, true><<<grid, block, 0, s>>>(p);
-  } else {
+  // Around the Infinity Cache's 256 MB plain loads are faster (us, non-temporal and plain: 117 MB 54 and 49, 268 MB 81 and
+  // 72), well above it non-temporal ones (470 MB 101 and 108, 537 MB 171 and 177).
+  auto go = [&](auto nt) {
+    constexpr bool kNt = decltype(nt)::value;
     switch (pl.mi) {
-      case 4: router_wgrad_kernel<4, false><<<grid, block, 0, s>>>(p); break;
-      case 8: router_wgrad_kernel<8, false><<<grid, block, 0, s>>>(p); break;
-      case 16: router_wgrad_kernel<16, false><<<grid, block, 0, s>>>(p); break;
-      default: router_wgrad_kernel<20, false><<<grid, block, 0, s>>>(p); break;
+      case 4: router_wgrad_kernel<4, false, kNt><<<grid, block, 0, s>>>(p); break;
+      case 8: router_wgrad_kernel<8, false, kNt><<<grid, block, 0, s>>>(p); break;
+      case 16: router_wgrad_kernel<16, false, kNt><<<grid, block, 0, s>>>(p); break;
+      default: router_wgrad_kernel<20, false, kNt><<<grid, block, 0, s>>>(p); break;
     }
-  }
+  };
+  if (K >= kWideK) router_wgrad_kernel<4, true, false><<<grid, block, 0, s>>>(p);
+  else if (M * K > 96 << 20) go(std::true_type{});
+  else go(std::false_type{});
   if (pl.s > 1) {
     router_wgrad_sum_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N * K / 4, 256))), dim3(256), 0, s>>>(planes, static_cast<int>(pl.s), N * K, out);
   }
