@@ -1929,9 +1929,8 @@ __global__ __launch_bounds__(256) void colmax_partial_kernel(const float *src, i
   }
 }
 
-// exp[c] = scale_exp(largest of part[0..S)[c]) (S <= 64: eight independent loads per round); kI8: clamped to
-// at most 127 (columns whose largest magnitude lies below 2^-112) and also written as int8 to exp8.
-template <bool kI8 = false>
+// exp[c] = scale_exp(largest of part[0..S)[c]) (S <= 64: eight independent loads per round), clamped to at most 127
+// (columns whose largest magnitude lies below 2^-112) and also written as int8 to exp8.
 __global__ __launch_bounds__(256) void colmax_final_kernel(const float *part, int S, int64_t C, int32_t *exp,
                                                            int8_t *exp8) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1944,14 +1943,9 @@ __global__ __launch_bounds__(256) void colmax_final_kernel(const float *part, in
 #pragma unroll
     for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
   }
-  if constexpr (kI8) {
-    const int e = min(scale_exp(m), 127);
-    exp[c] = e;
-    exp8[c] = static_cast<int8_t>(e);
-  } else {
-    (void)exp8;
-    exp[c] = scale_exp(m);
-  }
+  const int e = min(scale_exp(m), 127);
+  exp[c] = e;
+  exp8[c] = static_cast<int8_t>(e);
 }
 
 // Row-scaled fp16 copy for the tf32 router dgrad: one wavefront per row r of src [R, C] (C % 4 == 0), the row's
@@ -2393,7 +2387,7 @@ int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const 
     // Scale exponents of weight's columns and its fp16 copy, then grad_output's rows with their fp16 copy.
     colmax_partial_kernel<<<dim3(static_cast<uint32_t>(l.cb.xb), static_cast<uint32_t>(l.cb.S)), dim3(256), 0, s>>>(
         weight, K, N, l.cb.rps, l.cb.cg, part_b);
-    colmax_final_kernel<true><<<dim3(static_cast<uint32_t>(ceil_div(N, 256))), dim3(256), 0, s>>>(
+    colmax_final_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N, 256))), dim3(256), 0, s>>>(
         part_b, static_cast<int>(l.cb.S), N, col_e32, col_e8);
     const int64_t gb = std::max<int64_t>(1, std::min<int64_t>(ceil_div(K * N / 4, 256), 8192));
     tf32_to_f16_cols_kernel<<<dim3(static_cast<uint32_t>(gb)), dim3(256), 0, s>>>(weight, K, N, col_e32, b16);
