@@ -43,3 +43,21 @@ def test_row_id_map_one_launch_sizes(pkg, dev, T, E):
         assert torch.equal(got["expert_major_i32"].cpu().long(), row_em)
         assert torch.equal(got["expert_offsets"].cpu(), ref_torch.expert_offsets(rm))
         assert torch.equal(got["src_token"].cpu().long(), rm.t().nonzero()[:, 1])
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("T,E", [(63, 32), (255, 64), (257, 32), (1023, 96), (4097, 320), (16641, 64)])
+def test_row_id_map_paired_stores(pkg, dev, T, E, shift):
+    # Whole groups of 32 experts: token-major rows in pairs on a 16-byte aligned output, one at a time on another; nothing
+    # outside the output is written.
+    L = pkg._lib
+    g = torch.Generator().manual_seed(T + E)
+    rm = torch.rand(T, E, generator=g) < 0.1
+    m = rm.to(torch.uint8).to(dev)
+    buf = torch.full((T * E + 4,), -7, dtype=torch.int64, device=dev)
+    out = buf[2 + shift:2 + shift + T * E]
+    n = L.lib().moe_row_id_map_workspace_size(T, E)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    L.call("moe_row_id_map", m.data_ptr(), T, E, None, out.data_ptr(), None, None, None, 0, ws.data_ptr(), n, L.stream_handle())
+    assert torch.equal(out.view(T, E).cpu(), ref_torch.row_id_map(rm)[1])
+    assert (buf[:2 + shift] == -7).all() and (buf[2 + shift + T * E:] == -7).all()
