@@ -49,8 +49,7 @@ namespace moe {
 namespace {
 
 constexpr int kChunk = 64;                       // tokens per chunk = wave width (one ballot)
-constexpr int kThreads = 1024;                   // count / fill blocks (16 wavefronts; 512 measured
-                                                 // 16% slower at c5, 6% faster at case12)
+constexpr int kThreads = 1024;                   // count / fill blocks (16 wavefronts)
 constexpr int kWaves = kThreads / kWave;
 constexpr int kTileChunks = 4;                   // chunks per mask tile
 constexpr int kTile = kTileChunks * kChunk;      // 256 tokens per mask tile
@@ -99,9 +98,10 @@ __device__ __forceinline__ void tile_store(const u32x4 &v, uint8_t *tile, int nv
 }
 
 // Byte form for other E or alignments (one 0/1 byte per thread and step).
+template <int kT>
 __device__ __forceinline__ void tile_load_bytes(uint8_t *tile, const uint8_t *mask, int64_t E, int64_t t0,
                                                 int64_t t_lim, int64_t eg0, int eg_n) {
-  for (int i = threadIdx.x; i < kTile * kEG; i += kThreads) {
+  for (int i = threadIdx.x; i < kTile * kEG; i += kT) {
     const int r = i / kEG, c = i % kEG;
     uint8_t v = 0;
     if (c < eg_n && t0 + r < t_lim) v = mask[(t0 + r) * E + eg0 + c] != 0;
@@ -109,16 +109,18 @@ __device__ __forceinline__ void tile_load_bytes(uint8_t *tile, const uint8_t *ma
   }
 }
 
-// Mask bytes of this lane's token (row `row` of the tile) for the kEQ experts of part jq.
+// Mask bytes of this lane's token (row `row` of the tile) for the kN experts of part jq.
+template <int kN>
 struct LaneBytes {
-  uint32_t w[kEQ / 4];
+  uint32_t w[kN / 4];
   __device__ __forceinline__ bool operator()(int j) const { return ((w[j >> 2] >> (8 * (j & 3))) & 0xffu) != 0u; }
 };
-__device__ __forceinline__ LaneBytes lane_bytes(const uint8_t *tile, int row, int jq) {
-  const uint32_t *p = reinterpret_cast<const uint32_t *>(tile + row * kTileStride + jq * kEQ);
-  LaneBytes b;
+template <int kN>
+__device__ __forceinline__ LaneBytes<kN> lane_bytes(const uint8_t *tile, int row, int jq) {
+  const uint32_t *p = reinterpret_cast<const uint32_t *>(tile + row * kTileStride + jq * kN);
+  LaneBytes<kN> b;
 #pragma unroll
-  for (int q = 0; q < kEQ / 4; ++q) b.w[q] = p[q];
+  for (int q = 0; q < kN / 4; ++q) b.w[q] = p[q];
   return b;
 }
 
@@ -147,10 +149,10 @@ __global__ __launch_bounds__(kThreads) void rim_count_kernel(const uint8_t *mask
       tile_store(r, tile, nv);
       if (t0 + kTile < t_end) r = tile_fetch(mask, E, t0 + kTile, t_end, eg0, nv);
     } else {
-      tile_load_bytes(tile, mask, E, t0, t_end, eg0, eg_n);
+      tile_load_bytes<kThreads>(tile, mask, E, t0, t_end, eg0, eg_n);
     }
     __syncthreads();
-    const LaneBytes mb = lane_bytes(tile, c * kChunk + lane, jq);
+    const LaneBytes<kEQ> mb = lane_bytes<kEQ>(tile, c * kChunk + lane, jq);
 #pragma unroll
     for (int j = 0; j < kEQ; ++j) {
       if (jq * kEQ + j < eg_n) {
@@ -184,13 +186,17 @@ __device__ __forceinline__ int set_bytes(uint32_t v) { return __popc((((v & 0x7f
 // instructions of the part that follows the last barrier (both launches at 16384 tokens x 64 experts 11.2 -> 10.3 us,
 // x 320 26.0 -> 23.8, 32768 x 64 16.3 -> 14.5, 93 x 64 in one launch 5.8 -> 5.0). The other form has only single rows: with
 // both in one kernel E = 8 and 60 measured 0.1-0.3 us slower.
-template <bool kAlone, bool kWide>
-__global__ __launch_bounds__(kThreads) void rim_fill_kernel(const uint8_t *mask, int64_t T, int64_t E, int64_t L,
+// kT threads: 1024; 512 where the blocks are more than two for each CU (16384 tokens x 320 experts, 640 blocks, both
+// launches 23.8 -> 22.3 us; x 512 32.3 -> 26.6; 8192 x 1024 31.8 -> 26.5; 16384 x 304 without pairs 25.9 -> 24.0): three of
+// those share a CU. In one round the larger blocks are faster (16384 x 64 10.3 against 11.6, 4096 x 256 10.2 against 11.3).
+template <bool kAlone, bool kWide, int kT = kThreads>
+__global__ __launch_bounds__(kT) void rim_fill_kernel(const uint8_t *mask, int64_t T, int64_t E, int64_t L,
                                                             int64_t S, int64_t G, const int32_t *counts,
                                                             const int32_t *gsum, int64_t *row_em, int64_t *row_tm,
                                                             int32_t *row_em32, int32_t *expert_offsets,
                                                             int32_t *src_token, int64_t src_capacity, bool vec) {
-  constexpr int kParts = kThreads / kEG;  // threads per expert for the sums over super-chunks
+  constexpr int kWaves = kT / kWave, kQ = kWaves / kTileChunks, kEQ = kEG / kQ;
+  constexpr int kParts = kT / kEG;  // threads per expert for the sums over super-chunks
   constexpr int kPer = kMaxS / kParts;     // super-chunks per thread
   __shared__ __attribute__((aligned(16))) uint8_t tile[kTile * kTileStride];
   __shared__ int32_t out_tile[kTileChunks][kChunk * (kEG + 1)];
@@ -214,24 +220,24 @@ __global__ __launch_bounds__(kThreads) void rim_fill_kernel(const uint8_t *mask,
     // Rows before this group: the mask bytes of the experts below it.
     if (vec) {
       const int per = static_cast<int>(eg0 / 16);
-      for (int i = threadIdx.x; i < static_cast<int>(T) * per; i += kThreads) {
+      for (int i = threadIdx.x; i < static_cast<int>(T) * per; i += kT) {
         const int row = i / per;
         const u32x4 v = *reinterpret_cast<const u32x4 *>(mask + row * E + (i - row * per) * 16);
         part += set_bytes(v.x) + set_bytes(v.y) + set_bytes(v.z) + set_bytes(v.w);
       }
       tile_store(r, tile, nv);
     } else {
-      for (int i = threadIdx.x; i < static_cast<int>(T * eg0); i += kThreads) {
+      for (int i = threadIdx.x; i < static_cast<int>(T * eg0); i += kT) {
         const int row = i / static_cast<int>(eg0);
         part += mask[row * E + (i - row * eg0)] != 0;
       }
-      tile_load_bytes(tile, mask, E, t_begin, t_end, eg0, eg_n);
+      tile_load_bytes<kT>(tile, mask, E, t_begin, t_end, eg0, eg_n);
     }
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d);
     if (lane == 0) s_red[wave] = part;
     __syncthreads();
-    const LaneBytes mb = lane_bytes(tile, c * kChunk + lane, jq);
+    const LaneBytes<kEQ> mb = lane_bytes<kEQ>(tile, c * kChunk + lane, jq);
     int32_t n_mine = 0;
 #pragma unroll
     for (int j = 0; j < kEQ; ++j) {
@@ -311,11 +317,11 @@ __global__ __launch_bounds__(kThreads) void rim_fill_kernel(const uint8_t *mask,
       tile_store(r, tile, nv);
       if (t0 + kTile < t_end) r = tile_fetch(mask, E, t0 + kTile, t_end, eg0, nv);
     } else {
-      tile_load_bytes(tile, mask, E, t0, t_end, eg0, eg_n);
+      tile_load_bytes<kT>(tile, mask, E, t0, t_end, eg0, eg_n);
     }
     __syncthreads();
     // This lane's token of chunk c: its 8 mask bytes of quarter jq in a register.
-    const LaneBytes selected = lane_bytes(tile, c * kChunk + lane, jq);
+    const LaneBytes<kEQ> selected = lane_bytes<kEQ>(tile, c * kChunk + lane, jq);
     // Counts of chunk c for this wave's experts.
     int32_t my_cc = 0;
 #pragma unroll
@@ -475,9 +481,11 @@ int moe_row_id_map(const uint8_t *routing_map, int64_t T, int64_t E, int64_t *ro
   rim_count_kernel<<<grid, dim3(kThreads), 0, s>>>(routing_map, T, E, L, G, counts, gsum, vec);
   const int st = check_launch("moe_row_id_map(count)");
   if (st != MOE_OK) return st;
-  const auto fill = wide ? rim_fill_kernel<false, true> : rim_fill_kernel<false, false>;
-  fill<<<grid, dim3(kThreads), 0, s>>>(routing_map, T, E, L, S, G, counts, gsum, row_expert_major, row_token_major,
-                                       row_expert_major_i32, expert_offsets, src_token, src_capacity, vec);
+  const bool small = S * G > 2 * 256;  // two blocks for each CU
+  const auto fill = small ? (wide ? rim_fill_kernel<false, true, 512> : rim_fill_kernel<false, false, 512>)
+                          : (wide ? rim_fill_kernel<false, true> : rim_fill_kernel<false, false>);
+  fill<<<grid, dim3(small ? 512 : kThreads), 0, s>>>(routing_map, T, E, L, S, G, counts, gsum, row_expert_major, row_token_major,
+                                                     row_expert_major_i32, expert_offsets, src_token, src_capacity, vec);
   return check_launch("moe_row_id_map(fill)");
 }
 

@@ -61,3 +61,17 @@ def test_row_id_map_paired_stores(pkg, dev, T, E, shift):
     L.call("moe_row_id_map", m.data_ptr(), T, E, None, out.data_ptr(), None, None, None, 0, ws.data_ptr(), n, L.stream_handle())
     assert torch.equal(out.view(T, E).cpu(), ref_torch.row_id_map(rm)[1])
     assert (buf[:2 + shift] == -7).all() and (buf[2 + shift + T * E:] == -7).all()
+
+
+@pytest.mark.parametrize("T", [16129, 16384])
+@pytest.mark.parametrize("E", [256, 257, 288, 300, 304, 320])
+def test_row_id_map_more_than_one_round(pkg, dev, T, E):
+    # 64 (63 or 64) super-chunks: up to 8 expert groups make 512 blocks of 1024 threads, 9 and more take 512 threads.
+    g = torch.Generator().manual_seed(T + E)
+    rm = torch.rand(T, E, generator=g) < 0.03
+    row_em, row_tm = ref_torch.row_id_map(rm)
+    got = pkg.ops.row_id_map(rm.to(torch.uint8).to(dev), expert_major_i32=True, expert_offsets=True, src_rows=int(rm.sum()))
+    assert torch.equal(got["expert_major"].cpu(), row_em) and torch.equal(got["token_major"].cpu(), row_tm)
+    assert torch.equal(got["expert_major_i32"].cpu().long(), row_em)
+    assert torch.equal(got["expert_offsets"].cpu(), ref_torch.expert_offsets(rm))
+    assert torch.equal(got["src_token"].cpu().long(), rm.t().nonzero()[:, 1])
