@@ -195,7 +195,9 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         if (st + k < steps) {
-          wait_vm_n<kDma + 16>();
+          // (kWide: a load that no lane of a wavefront takes is not issued, so the operations in flight cannot be counted.)
+          if constexpr (kWide) wait_dma();
+          else wait_vm_n<kDma + 16>();
           barrier();  // stage st + k has landed, and every wavefront is done with the stage before
           dma(st + k + 2);
           convert(buf[(2 * k) % 3]);

@@ -215,3 +215,20 @@ def test_router_dgrad_tf32_edges(pkg, dev, M, K, N):
     excess = (buf[1:M + 1].cpu().double() - a @ b).abs() - (1e-4 * (a.abs() @ b.abs()) + 2.0 ** -126)
     assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
     assert bool((buf[0] == 3.0).all()) and bool((buf[M + 1] == 3.0).all()), "stored outside grad_input"
+
+
+@pytest.mark.parametrize("M", [1, 33])
+def test_router_wgrad_tf32_rows_of_64_bit_offsets(pkg, dev, M):
+    # Rows of inp so long that 64 of them take 64-bit addresses, whose loads are left out where a wavefront has no row
+    # (M = 1: 31 of 32, and the second half of the stage) or no column (the last tile has 8): grad_output's tile is
+    # still complete in LDS before any wavefront multiplies it. Reference: float64 on the device, the bound of this file.
+    N, K = 8, (1 << 22) + 8
+    g = torch.Generator(device=dev).manual_seed(M)
+    go = torch.randn(M, N, generator=g, device=dev)
+    x = torch.randn(M, K, generator=g, device=dev)
+    got = pkg.ops.router_wgrad_tf32(go, x)
+    a, b = ref_torch.round_tf32_rne(go).double(), ref_torch.round_tf32_rne(x)
+    for at in range(0, K, 1 << 20):
+        bk = b[:, at:at + (1 << 20)].double()
+        err = (got[:, at:at + (1 << 20)].double() - a.t() @ bk).abs()
+        assert bool((err <= 1e-4 * (a.abs().t() @ bk.abs()) + 1e-5).all()), f"columns from {at}: worst error {err.max().item():.3e}"
