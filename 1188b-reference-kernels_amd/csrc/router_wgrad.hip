@@ -8,9 +8,10 @@
 //     loads two neighbouring columns of those 8 rows (8 bytes each, 128 contiguous bytes per row over 16 lanes) holds
 //     the fragments of two blocks, the even columns and the odd ones: no LDS, no transpose, no fp16 copy in memory;
 //   * the columns' scales are found on the way: a lane compares its magnitudes with the largest its column's scale
-//     takes (one ballot per 32 rows); only when one exceeds it (in the first rows, then rarely: the scale leaves a
-//     factor of 8) the column's maximum is formed across the lanes, and the sums so far, whose column is the lane's
-//     own, are multiplied by the change, a power of two;
+//     takes (one ballot per 32 rows); only when one exceeds it (in the first rows, then rarely) the column's maximum is
+//     formed across the lanes and scaled into [2^14, 2^15), and the sums so far, whose column is the lane's own, are
+//     multiplied by the change, a power of two. The scale holds up to fp16's largest value, so it is never below the
+//     one that the column's largest magnitude as a whole would take, and small values keep as many bits;
 //   * the small operand (grad_output, transposed and scaled in fp16 by a kernel before) comes through a ring of three
 //     LDS stages of 64 reduction rows, shared by the 8 wavefronts (256 columns);
 //   * M is cut into chunks so that there is a unit for every CU; the units of one XCD share a chunk, whose part of the
@@ -37,7 +38,7 @@ typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
 constexpr int kColsWave = 32, kColsTile = 256;
 constexpr int kRowB = kBK * 2;  // 128 bytes: one row of the small operand in a stage
 constexpr int64_t kWideK = int64_t(1) << 22;
-constexpr int kHeadroom = 3;    // a new scale puts the largest magnitude into [2^11, 2^12)
+constexpr float kF16Max = 65504.f;
 
 __device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
 
@@ -145,9 +146,9 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
         m = fmaxf(m, __shfl_xor(m, 16));
         m = fmaxf(m, __shfl_xor(m, 32));
         if (m >= most[j]) {
-          const int ne = scale_exp(m) - kHeadroom, d = ne - e[j];
+          const int ne = scale_exp(m), d = ne - e[j];
           e[j] = ne;
-          most[j] = __builtin_ldexpf(1.f, 15 - ne);
+          most[j] = __builtin_ldexpf(kF16Max, -ne);  // (tf32 rounding takes no value below it past it)
 #pragma unroll
           for (int i = 0; i < kMI; ++i)
 #pragma unroll

@@ -407,11 +407,12 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  * operands rounded to tf32 (round_tf32_rne, :51-58), products accumulated in
  * fp32, fp32 out.
  *   Both run on the fp16 matrix cores: a tf32 value has fp16's 11 significant
- *     bits; each operand row or column along which the sum runs is scaled by a
- *     power of two that brings its largest magnitude into [2^11, 2^15), so its
- *     values are fp16 values (exactly, unless 2^25 or more below that largest
- *     one: then within 2^-36 of it), the products are exact in fp32, and the
- *     sums are scaled back exactly (unless the result is an fp32 subnormal);
+ *     bits; each operand row or column along which the sum runs is scaled by
+ *     the power of two that brings its largest magnitude into [2^14, 2^15),
+ *     so its values are fp16 values (exactly, unless 2^29 or more below that
+ *     largest one: then within 2^-38 of it), the products are exact in fp32,
+ *     and the sums are scaled back exactly (unless the result is an fp32
+ *     subnormal);
  *     the scale comes from the largest finite magnitude (Inf and NaN entries
  *     stay Inf and NaN), a row or column with no finite nonzero value keeps
  *     scale 1 (dgrad: one whose largest is below 2^-112 takes 2^127).
@@ -419,8 +420,9 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  *     grad_output scaled per row, weight per column, the scales undone in the
  *     GEMM's epilogue.
  *   wgrad: grad_weight [N, K] = tf32(grad_output [M, N])^T @ tf32(inp [M, K]):
- *     both scaled per column; inp's scales are found as its rows stream by, and
- *     the sums so far follow a scale that changes.
+ *     both scaled per column; inp's scales are found as its rows stream by (the
+ *     largest magnitude so far, at most fp16's largest value), and the sums so
+ *     far follow a scale that changes.
  * Limits: the column counts (K and N) % 8 == 0; dgrad 3K, N < 2^22 and
  *   3K*N < 2^30; wgrad M*N, M*K, N*K < 2^30; 16-byte aligned tensors.
  * Workspace: the *_workspace_size bytes, 256-byte aligned (dgrad: the fp16

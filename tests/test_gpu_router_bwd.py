@@ -232,3 +232,28 @@ def test_router_wgrad_tf32_rows_of_64_bit_offsets(pkg, dev, M):
         bk = b[:, at:at + (1 << 20)].double()
         err = (got[:, at:at + (1 << 20)].double() - a.t() @ bk).abs()
         assert bool((err <= 1e-4 * (a.abs().t() @ bk.abs()) + 1e-5).all()), f"columns from {at}: worst error {err.max().item():.3e}"
+
+
+def test_router_wgrad_tf32_small_values_beside_a_large_one(pkg, dev):
+    # Column 5 of inp holds 2^27 in its first row and values of [1, 2) below, 2^27 to 2^28 smaller: scaled by the power
+    # of two that brings the large one to 2^14 they are fp16 normal numbers, so they keep all 11 significant bits. The
+    # first 32 outputs have grad_output 0 in the large one's row and see the small ones alone; the bound is that of a
+    # sum of M exact products in fp32, M 2^-24 sum |a b| over those products.
+    M, N, K = 120, 64, 264
+    g = torch.Generator().manual_seed(17)
+    go = torch.randn(M, N, generator=g)
+    x = torch.randn(M, K, generator=g)
+    x[:, 5] = (1 + torch.rand(M, generator=g)) * torch.sign(torch.randn(M, generator=g))
+    x[0, 5] = 2.0 ** 27
+    go[0, :32] = 0.0
+    # columns that grow up to the largest value that their first scale takes, and past it
+    x[:, 6] = 1.0
+    x[40, 6] = 65504.0 / 2 ** 14
+    x[:, 7] = 1.0
+    x[40, 7] = 65520.0 / 2 ** 14
+    got = pkg.ops.router_wgrad_tf32(go.to(dev), x.to(dev)).cpu().double()
+    a, b = ref_torch.round_tf32_rne(go).double(), ref_torch.round_tf32_rne(x).double()
+    err = (got - a.t() @ b).abs()
+    bound = M * 2.0 ** -24 * (a.abs().t() @ b.abs())
+    assert bool((err[:32] <= bound[:32]).all()), f"worst err/bound {(err[:32] / bound[:32]).max().item():.1f}"
+    assert bool((err[:, 6:8] <= bound[:, 6:8]).all())
