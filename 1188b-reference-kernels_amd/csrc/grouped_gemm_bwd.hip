@@ -2449,13 +2449,14 @@ int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const 
 namespace {
 
 // Workspace of the tf32 wgrad (byte offsets, each 256-byte aligned): the transposed fp16 copy of grad_output, its
-// scale exponents, its column-max slabs, and the fp32 planes of the reduction chunks (none for one chunk). Its size is
+// scale exponents, its column-max slabs, and the fp32 planes of the reduction chunks with the exponents of their columns
+// (none for one chunk). Its size is
 // never below `agreed`, what callers that sized their workspaces once were told: fp16 copies of both operands, both
 // operands' exponents and column-max slabs, and the planes of chunks of 512 rows or more.
 struct WgradTf32Layout {
   moe::RouterWgradPlan pl;
   moe::ColmaxPlan ca;
-  size_t rows, exp, part, planes, total;
+  size_t rows, exp, part, col_exp, planes, total;
 };
 WgradTf32Layout wgrad_tf32_layout(int64_t M, int64_t N, int64_t K) {
   using moe::align_up;
@@ -2471,6 +2472,7 @@ WgradTf32Layout wgrad_tf32_layout(int64_t M, int64_t N, int64_t K) {
   l.rows = take(static_cast<size_t>(moe::ceil_div(M, 64) * 64) * N * 2);
   l.exp = take(static_cast<size_t>(N) * 4);
   l.part = take(static_cast<size_t>(l.ca.S) * N * 4);
+  l.col_exp = take(l.pl.s > 1 ? static_cast<size_t>(l.pl.s) * K * 4 : 0);
   l.planes = take(l.pl.s > 1 ? static_cast<size_t>(l.pl.s) * N * K * 4 : 0);
   const int64_t tiles = moe::ceil_div(N, 256) * moe::ceil_div(K, 256);
   int64_t chunks = 1;
@@ -2527,7 +2529,8 @@ int moe_router_wgrad_tf32(const float *grad_output, int64_t M, int64_t N, const 
   colmax_partial_kernel<<<dim3(static_cast<uint32_t>(l.ca.xb), static_cast<uint32_t>(l.ca.S)), dim3(256), 0, s>>>(
       grad_output, M, N, l.ca.rps, l.ca.cg, part);
   launch_router_wgrad_rows(grad_output, M, N, part, static_cast<int>(l.ca.S), rows, exp, s);
-  launch_router_wgrad(l.pl, rows, exp, inp, M, N, K, reinterpret_cast<float *>(w + l.planes), grad_weight, s);
+  launch_router_wgrad(l.pl, rows, exp, inp, M, N, K, reinterpret_cast<float *>(w + l.planes), reinterpret_cast<int32_t *>(w + l.col_exp),
+                      grad_weight, s);
   return check_launch(fn);
 }
 

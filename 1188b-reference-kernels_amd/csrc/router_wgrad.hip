@@ -15,7 +15,8 @@
 //   * the small operand (grad_output, transposed and scaled in fp16 by a kernel before) comes through a ring of three
 //     LDS stages of 64 reduction rows, shared by the 8 wavefronts (256 columns);
 //   * M is cut into chunks so that there is a unit for every CU; the units of one XCD share a chunk, whose part of the
-//     small operand then stays in its L2. The planes of the chunks are added in order.
+//     small operand then stays in its L2. The planes of the chunks stay scaled, each column with its chunk's exponent;
+//     they are brought to the column's smallest exponent, added in order and scaled back once.
 // Measured (MI355X, 16384 x 320 x 8192, us): 395 -> 171 for the whole call; the GEMM 120-134 (4.0-4.5 TB/s of inp; 150 without the multiplications and conversions, so it is the loads), the
 // planes' sum 16, grad_output's maxima and copy 17. Before: column maxima of inp 90, its fp16 copy 180, a GEMM on the
 // copies 143, the sum 10. 16384 x 64 x 7168: 307 -> 101; 4096 x 128 x 7168: 98 -> 49; 100 x 64 x 7168: 39 -> 19.
@@ -33,12 +34,14 @@ using namespace gemm;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
 
 constexpr int kColsWave = 32, kColsTile = 256;
 constexpr int kRowB = kBK * 2;  // 128 bytes: one row of the small operand in a stage
 constexpr int64_t kWideK = int64_t(1) << 22;
 constexpr float kF16Max = 65504.f;
+constexpr int kNoExp = 1 << 20;  // a column without a finite nonzero value yet: its sums are 0, Inf or NaN, whatever the scale
 
 __device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
 
@@ -46,14 +49,16 @@ struct WgradArgs {
   const uint16_t *rows;  // [N, M64] fp16
   const int32_t *exp;    // [N]
   const float *inp;      // [M, K]
-  float *out;            // planes [s, N, K]
+  float *out;            // planes [s, N, K], or (one chunk) the result
+  int32_t *col_exp;      // the planes' column exponents [s, K]
   int64_t M, M64, N, K;
   int64_t chunk;         // reduction rows of a chunk
   int col_tiles, row_tiles, units;
 };
 
 // kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets). kNt: non-temporal loads of it.
-template <int kMI, bool kWide, bool kNt>
+// kOne: one chunk, whose sums are scaled back here.
+template <int kMI, bool kWide, bool kNt, bool kOne>
 __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
   constexpr int kStage = kMI * 16 * kRowB;
   constexpr int kSlots = 3;
@@ -126,7 +131,7 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
   f32x4 acc[kMI][2];
 #pragma unroll
   for (int i = 0; i < kMI; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int e[2] = {0, 0};             // the columns' scale exponents
+  int e[2] = {kNoExp, kNoExp};   // the columns' scale exponents
   // Magnitudes below it fit the scale; at first the smallest there is, which only zeros are below.
   float most[2] = {__uint_as_float(1u), __uint_as_float(1u)};
   f16x8 fb[2];
@@ -220,16 +225,22 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
   // acc[i][j] register t: row n0 + 16 i + 4 q + t, column col + j.
   float *const out = p.out + (static_cast<int64_t>(chunk) * p.N + n0) * p.K;
   if (col < p.K) {
+    if (!kOne && n0 == 0 && q == 0) {
+      *reinterpret_cast<u32x2 *>(p.col_exp + chunk * p.K + col) = u32x2{static_cast<uint32_t>(e[0]), static_cast<uint32_t>(e[1])};
+    }
 #pragma unroll
     for (int i = 0; i < kMI; ++i) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int r = i * 16 + q * 4 + t;
         if (n0 + r < p.N) {
-          const int er = p.exp[n0 + r];
-          const u32x2 v = {__float_as_uint(__builtin_ldexpf(acc[i][0][t], -(er + e[0]))),
-                           __float_as_uint(__builtin_ldexpf(acc[i][1][t], -(er + e[1])))};
-          *reinterpret_cast<u32x2 *>(out + static_cast<int64_t>(r) * p.K + col) = v;
+          float v0 = acc[i][0][t], v1 = acc[i][1][t];
+          if constexpr (kOne) {
+            const int er = p.exp[n0 + r];
+            v0 = __builtin_ldexpf(v0, -(er + e[0]));
+            v1 = __builtin_ldexpf(v1, -(er + e[1]));
+          }
+          *reinterpret_cast<u32x2 *>(out + static_cast<int64_t>(r) * p.K + col) = u32x2{__float_as_uint(v0), __float_as_uint(v1)};
         }
       }
     }
@@ -285,13 +296,31 @@ __global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src
   }
 }
 
-// out[i] = sum over s of planes[s][i], s ascending (n % 4 == 0).
-__global__ __launch_bounds__(256) void router_wgrad_sum_kernel(const float *planes, int s, int64_t n, float *out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i * 4 >= n) return;
-  f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes) + i);
-  for (int k = 1; k < s; ++k) a += __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes + k * n) + i);
-  reinterpret_cast<f32x4 *>(out)[i] = a;
+// out[n][k] = 2^-(exp[n] + E[k]) sum over s of 2^(E[k] - col_exp[s][k]) planes[s][n][k], s ascending, E[k] the smallest
+// col_exp[.][k] (the smallest so far on the way): no plane is made larger, and none leaves the scaled range before the
+// total does. N K is a multiple of 64 and below 2^30.
+__global__ __launch_bounds__(256) void router_wgrad_sum_kernel(const float *planes, int s, int64_t N, int64_t K, const int32_t *exp,
+                                                               const int32_t *col_exp, float *out) {
+  const uint32_t quads = static_cast<uint32_t>(K / 4), i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t n = i / quads, c = (i - n * quads) * 4;
+  if (n >= static_cast<uint32_t>(N)) return;
+  f32x4 sum = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes) + i);
+  i32x4 least = *reinterpret_cast<const i32x4 *>(col_exp + c);
+#pragma unroll 4
+  for (int k = 1; k < s; ++k) {
+    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(planes + k * N * K) + i);
+    const i32x4 v = *reinterpret_cast<const i32x4 *>(col_exp + k * K + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int e = min(least[j], v[j]);
+      sum[j] = __builtin_ldexpf(sum[j], e - least[j]) + __builtin_ldexpf(a[j], e - v[j]);
+      least[j] = e;
+    }
+  }
+  const int er = exp[n];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum[j] = __builtin_ldexpf(sum[j], -(er + least[j]));
+  reinterpret_cast<f32x4 *>(out)[i] = sum;
 }
 
 }  // namespace
@@ -320,12 +349,13 @@ void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, co
 }
 
 void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const int32_t *exp, const float *inp, int64_t M, int64_t N,
-                         int64_t K, float *planes, float *out, hipStream_t s) {
+                         int64_t K, float *planes, int32_t *col_exp, float *out, hipStream_t s) {
   WgradArgs p;
   p.rows = rows;
   p.exp = exp;
   p.inp = inp;
   p.out = pl.s > 1 ? planes : out;
+  p.col_exp = col_exp;
   p.M = M;
   p.M64 = ceil_div(M, 64) * 64;
   p.N = N;
@@ -338,20 +368,23 @@ void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const 
   const dim3 grid(static_cast<uint32_t>((units + 7) / 8 * 8)), block(512);
   // Around the Infinity Cache's 256 MB plain loads are faster (us, non-temporal and plain: 117 MB 54 and 49, 268 MB 81 and
   // 72), well above it non-temporal ones (470 MB 101 and 108, 537 MB 171 and 177).
-  auto go = [&](auto nt) {
-    constexpr bool kNt = decltype(nt)::value;
+  auto go = [&](auto nt, auto one) {
+    constexpr bool kNt = decltype(nt)::value, kOne = decltype(one)::value;
     switch (pl.mi) {
-      case 4: router_wgrad_kernel<4, false, kNt><<<grid, block, 0, s>>>(p); break;
-      case 8: router_wgrad_kernel<8, false, kNt><<<grid, block, 0, s>>>(p); break;
-      case 16: router_wgrad_kernel<16, false, kNt><<<grid, block, 0, s>>>(p); break;
-      default: router_wgrad_kernel<20, false, kNt><<<grid, block, 0, s>>>(p); break;
+      case 4: router_wgrad_kernel<4, false, kNt, kOne><<<grid, block, 0, s>>>(p); break;
+      case 8: router_wgrad_kernel<8, false, kNt, kOne><<<grid, block, 0, s>>>(p); break;
+      case 16: router_wgrad_kernel<16, false, kNt, kOne><<<grid, block, 0, s>>>(p); break;
+      default: router_wgrad_kernel<20, false, kNt, kOne><<<grid, block, 0, s>>>(p); break;
     }
   };
-  if (K >= kWideK) router_wgrad_kernel<4, true, false><<<grid, block, 0, s>>>(p);
-  else if (M * K > 96 << 20) go(std::true_type{});
-  else go(std::false_type{});
+  const bool nt = M * K > 96 << 20;
+  if (K >= kWideK) router_wgrad_kernel<4, true, false, true><<<grid, block, 0, s>>>(p);  // (fewer than 256 rows: one chunk)
+  else if (pl.s == 1) go(std::false_type{}, std::true_type{});
+  else if (nt) go(std::true_type{}, std::false_type{});
+  else go(std::false_type{}, std::false_type{});
   if (pl.s > 1) {
-    router_wgrad_sum_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N * K / 4, 256))), dim3(256), 0, s>>>(planes, static_cast<int>(pl.s), N * K, out);
+    router_wgrad_sum_kernel<<<dim3(static_cast<uint32_t>(ceil_div(N * K / 4, 256))), dim3(256), 0, s>>>(
+        planes, static_cast<int>(pl.s), N, K, exp, col_exp, out);
   }
 }
 

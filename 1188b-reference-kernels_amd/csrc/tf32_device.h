@@ -42,9 +42,10 @@ RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K);
 // by 2^exp[n]; exp[n] from the column maxima of `slabs` slabs (part [slabs, N]).
 void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, const float *part, int slabs, uint16_t *rows, int32_t *exp,
                               hipStream_t s);
-// planes[chunk][N][K] (s == 1: the result itself), then their sum in chunk order.
+// planes[chunk][N][K], scaled by exp and col_exp[chunk][K], then their sum in chunk order, scaled back (s == 1: the result
+// itself, neither is used).
 void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const int32_t *exp, const float *inp, int64_t M, int64_t N,
-                         int64_t K, float *planes, float *out, hipStream_t s);
+                         int64_t K, float *planes, int32_t *col_exp, float *out, hipStream_t s);
 
 // ---- router dgrad (router_dgrad.hip): reductions of at most 320
 

@@ -422,7 +422,8 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  *   wgrad: grad_weight [N, K] = tf32(grad_output [M, N])^T @ tf32(inp [M, K]):
  *     both scaled per column; inp's scales are found as its rows stream by (the
  *     largest magnitude so far, at most fp16's largest value), and the sums so
- *     far follow a scale that changes.
+ *     far follow a scale that changes. The sums of reduction chunks are added
+ *     while scaled, so only the total has to be in fp32's range.
  * Limits: the column counts (K and N) % 8 == 0; dgrad 3K, N < 2^22 and
  *   3K*N < 2^30; wgrad M*N, M*K, N*K < 2^30; 16-byte aligned tensors.
  * Workspace: the *_workspace_size bytes, 256-byte aligned (dgrad: the fp16
@@ -430,7 +431,7 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  *   reduction values), the row and column exponents and, for longer
  *   reductions, the column-max slabs; wgrad: the transposed fp16 copy of grad_output, its
  *   columns' exponents and column-max slabs, and the fp32 planes of the
- *   reduction chunks where there are several; at least the size of an fp16
+ *   reduction chunks with their columns' exponents where there are several; at least the size of an fp16
  *   copy of both operands with their exponents, slabs and planes). */
 size_t moe_router_dgrad_tf32_workspace_size(int64_t M, int64_t K, int64_t N);
 int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const float *weight, int64_t N,

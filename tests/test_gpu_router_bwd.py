@@ -257,3 +257,22 @@ def test_router_wgrad_tf32_small_values_beside_a_large_one(pkg, dev):
     bound = M * 2.0 ** -24 * (a.abs().t() @ b.abs())
     assert bool((err[:32] <= bound[:32]).all()), f"worst err/bound {(err[:32] / bound[:32]).max().item():.1f}"
     assert bool((err[:, 6:8] <= bound[:, 6:8]).all())
+
+
+def test_router_wgrad_tf32_sums_of_chunks_beyond_fp32(pkg, dev):
+    # The reduction of 512 rows runs in chunks. Their sums alone lie beyond fp32's range (64 products of 2^126 and more
+    # of one sign), the total does not: the chunks are added while scaled. Columns that are zero in all chunks but one,
+    # with values near the smallest there are, and a column of zeros check what a chunk without a scale adds.
+    M, N, K = 512, 64, 256
+    go = torch.full((M, N), 2.0 ** 60)
+    x = torch.full((M, K), 2.0 ** 66)
+    x[M // 2:] *= -1.0
+    x[M - 1] *= 0.5              # total: 2^125
+    x[:, 1] = 0.0
+    x[M - 1, 1] = 2.0 ** -136    # the smallest value that the rounding to tf32 leaves, an fp32 subnormal
+    x[:, 2] = 0.0
+    x[0, 2] = -(2.0 ** -133)
+    x[:, 3] = 0.0
+    got = pkg.ops.router_wgrad_tf32(go.to(dev), x.to(dev)).cpu().double()
+    ref = go.double().t() @ x.double()  # all values are tf32 values
+    assert torch.equal(got, ref), (got[0, :5], ref[0, :5])
