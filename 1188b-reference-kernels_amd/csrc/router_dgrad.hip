@@ -29,19 +29,22 @@ using namespace gemm;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
-typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 constexpr int kRowsStage = 64, kColsWave = 64, kColsTile = 512;
+// Rows' exponents as bytes: scale_exp is -113 to 163, and a row whose largest magnitude is below 2^-128 (above 142) is as
+// exact with 142: its values, multiples of 2^-149, become multiples of 2^-7 below 2^14.
+constexpr int kExpBias = 15, kExpMost = 127 + kExpBias;
 
 struct DgradArgs {
-  const uint16_t *a;    // [M64, 64 kKS2] fp16: scaled rows of grad_output, zeros past K and M
-  const uint16_t *b;    // [N, 64 kKS2] fp16: scaled columns of weight
-  const int32_t *a_exp; // [M64]
+  const uint16_t *a;    // [M, K] fp16: scaled rows of grad_output
+  const uint16_t *b;    // [N, K] fp16: scaled columns of weight
+  const int8_t *a_exp;  // [M rounded up to 4]: exponents, kExpBias less
   const int32_t *b_exp; // [N]
   float *out;
   int64_t M, N;
+  int K;                // (a row's 64 kKS2 values past K are zeros)
   int64_t chunk;        // rows of a unit (a multiple of 64)
   int col_tiles, units;
 };
@@ -50,7 +53,7 @@ struct DgradArgs {
 template <int kKS2>
 __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
   constexpr int kKS = 2 * kKS2;                  // MFMAs per block
-  constexpr int kRowB = 128 * kKS2;              // bytes of a row
+  constexpr int kRowB = 128 * kKS2;              // bytes of a row in LDS
   constexpr int kStage = kRowsStage * kRowB;     // 8 kKS2 KiB
   constexpr int kExp = kRowsStage * 4;           // the rows' exponents
   constexpr int kSlots = 3;
@@ -70,26 +73,31 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
   const int64_t m0 = static_cast<int64_t>(u / p.col_tiles) * p.chunk, m1 = min(p.M, m0 + p.chunk);
   const int stages = static_cast<int>((m1 - m0 + kRowsStage - 1) / kRowsStage);
 
-  // ---- rows: block wave + 8 j of a stage; 16-byte chunks of a row are XORed with the row within each 128 bytes. The
-  // offsets are formed anew for each stage (from a lane index the compiler takes for another): the registers are the
-  // weight's.
+  // ---- rows: block wave + 8 j of a stage; 16-byte chunks of a row are XORed with the row within each 128 bytes, those past
+  // K and rows past M read zeros. The offsets are formed anew for each stage (from a lane index the compiler takes for
+  // another): the registers are the weight's.
+  const int row_bytes = p.K * 2;
   auto dma = [&](int st) {
     const int sc = min(st, stages - 1);  // past the last stage the last one again, into a slot nothing reads any more
     const int64_t m = m0 + static_cast<int64_t>(sc) * kRowsStage;
     const int slot = st % kSlots;
     if (wave == 0) {
 #if defined(__HIP_DEVICE_COMPILE__)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.a_exp + m, kExp), (lds_void *)(uintptr_t)(lds_exp + slot * kExp), 4, lane * 4, 0, 0, 0);
+      const uint32_t bytes = static_cast<uint32_t>(min<int64_t>(kRowsStage, (p.M - m + 3) & ~int64_t(3)));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.a_exp + m, bytes), (lds_void *)(uintptr_t)(lds_exp + slot * kExp), 4, lane * 4, 0, 0, 0);
 #endif
     }
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a + m * (kRowB / 2), kStage);
+    const __amdgpu_buffer_rsrc_t ra =
+        make_rsrc(p.a + m * p.K, static_cast<uint32_t>(static_cast<int>(min<int64_t>(kRowsStage, p.M - m)) * row_bytes));
     int ln = lane;
     asm volatile("" : "+v"(ln));
 #pragma unroll
     for (int j = 0; j < kDma; ++j) {
       const int at = (wave + 8 * j) * 64 + ln;  // chunk of the stage, as it lies in LDS
       const int r = at / (8 * kKS2), c = at % (8 * kKS2);
-      dma16b(ra, (lds_void *)(uintptr_t)(lds + slot * kStage + (wave + 8 * j) * 1024), r * kRowB + ((c & ~7) | ((c ^ r) & 7)) * 16, 0);
+      const int from = ((c & ~7) | ((c ^ r) & 7)) * 16;
+      dma16b(ra, (lds_void *)(uintptr_t)(lds + slot * kStage + (wave + 8 * j) * 1024),
+             from < row_bytes ? r * row_bytes + from : static_cast<int>(kNoAccess), 0);
     }
   };
   dma(0);
@@ -98,14 +106,26 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
   // ---- this wavefront's columns
   const int64_t n0 = static_cast<int64_t>(ct) * kColsTile + wave * kColsWave + 4 * c16;
   const bool in = n0 < p.N;  // N % 8 == 0: a lane's four columns are all valid or all past N
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b, static_cast<uint32_t>(p.N) * static_cast<uint32_t>(row_bytes));  // 3 K N < 2^30
   f16x8 fb[kKS][4];
   int eb[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int64_t n = in ? n0 + j : 0;
-    eb[j] = p.b_exp[n];
+    eb[j] = p.b_exp[n] + kExpBias;
 #pragma unroll
-    for (int ks = 0; ks < kKS; ++ks) fb[ks][j] = *reinterpret_cast<const f16x8 *>(p.b + n * (kRowB / 2) + ks * 32 + q * 8);
+    for (int ks = 0; ks < kKS; ++ks) {
+      const int k = ks * 32 + q * 8;
+#if defined(__HIP_DEVICE_COMPILE__)
+      fb[ks][j] = __builtin_bit_cast(
+          f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                     rb, k < p.K ? static_cast<int>(n) * row_bytes + k * 2 : static_cast<int>(kNoAccess), 0, 0));
+#else
+      (void)k;
+      (void)rb;
+      fb[ks][j] = f16x8{};
+#endif
+    }
   }
   const uint32_t ld = static_cast<uint32_t>(p.N) * 4u;
   const uint32_t o_lane = in ? static_cast<uint32_t>(4 * q) * ld + static_cast<uint32_t>(n0) * 4u : kNoAccess;
@@ -129,7 +149,7 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
         return *reinterpret_cast<const lds_f16x8 *>((uintptr_t)((base ^ ((ks & 1) << 6)) + i * 16 * kRowB + (ks >> 1) * 128));
       };
       fa[0] = read(0);
-      const i32x4 ea = *reinterpret_cast<const lds_i32x4 *>((uintptr_t)(ebase + (i * 16 + 4 * q) * 4));
+      const uint32_t ea = *reinterpret_cast<const lds_u32 *>((uintptr_t)(ebase + i * 16 + 4 * q));  // four rows' bytes
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
         if (ks + 1 < kKS) fa[(ks + 1) & 1] = read(ks + 1);
@@ -142,8 +162,9 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         u32x4 v;
+        const int er = static_cast<int8_t>(ea >> (8 * t));
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(__builtin_ldexpf(acc[j][t], -(ea[t] + eb[j])));
+        for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(__builtin_ldexpf(acc[j][t], -(er + eb[j])));
 #if defined(__HIP_DEVICE_COMPILE__)
         __builtin_amdgcn_raw_buffer_store_b128(v, ro, static_cast<int>(in ? o_lane + static_cast<uint32_t>(i * 16 + t) * ld : kNoAccess), 0, 0);
 #else
@@ -159,11 +180,11 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
 }
 
 // Both operands in one launch. Blocks [0, wb): 64 columns of weight [K, N] each, all K <= 64 kV / 4 rows: its columns'
-// largest finite magnitudes, their exponents, the scaled columns as rows of b (kp long, zeros past K). The other blocks:
-// four rows of grad_output each, one per wavefront (rows past M: zeros and exponent 0).
+// largest finite magnitudes, their exponents, the scaled columns as rows of b. The other blocks: four rows of grad_output
+// each, one per wavefront.
 template <int kV>
-__global__ __launch_bounds__(256) void router_dgrad_prepare_kernel(const float *w, const float *go, int64_t M, int64_t M64, int K, int64_t N,
-                                                                   int kp, int wb, uint16_t *a, uint16_t *bt, int32_t *a_exp, int32_t *b_exp) {
+__global__ __launch_bounds__(256) void router_dgrad_prepare_kernel(const float *w, const float *go, int64_t M, int K, int64_t N, int wb,
+                                                                   uint16_t *a, uint16_t *bt, int8_t *a_exp, int32_t *b_exp) {
   constexpr int kRows = 16 * kV;              // rows of weight held by a block
   constexpr int kPitch = kRows + 8;           // LDS row of a column, in values (16-byte rows; a bank offset per column)
   __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kPitch];
@@ -202,39 +223,39 @@ __global__ __launch_bounds__(256) void router_dgrad_prepare_kernel(const float *
         tile[(c + k) * kPitch + r0 + 16 * i] =
             __builtin_bit_cast(uint16_t, static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(v[i][k])), e[k])));
     __syncthreads();
-    const int per = kp / 8;  // 16-byte pieces of a column
+    const int per = K / 8;  // 16-byte pieces of a column
     for (int i = t; i < 64 * per; i += 256) {
       const int n = i / per, k = i - n * per;
-      if (n0 + n < N) *reinterpret_cast<u32x4 *>(bt + (n0 + n) * kp + k * 8) = *reinterpret_cast<const u32x4 *>(&tile[n * kPitch + k * 8]);
+      if (n0 + n < N) *reinterpret_cast<u32x4 *>(bt + (n0 + n) * K + k * 8) = *reinterpret_cast<const u32x4 *>(&tile[n * kPitch + k * 8]);
     }
     return;
   }
   const int64_t m = static_cast<int64_t>(blockIdx.x - wb) * 4 + t / kWave;
   const int lane = t % kWave;
-  if (m >= M64) return;
+  if (m >= M) return;
   constexpr int kU = (kRows + 255) / 256;  // 4 values a lane at a time
   u32x4 v[kU];
   float mx = 0.f;
 #pragma unroll
   for (int i = 0; i < kU; ++i) {
     const int k = (lane + i * kWave) * 4;
-    v[i] = m < M && k < K ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(go + m * K + k)) : u32x4{0u, 0u, 0u, 0u};
+    v[i] = k < K ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(go + m * K + k)) : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int j = 0; j < 4; ++j) mx = fmaxf(mx, finite_abs(__uint_as_float(v[i][j])));
   }
 #pragma unroll
   for (int d = kWave / 2; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-  const int e = scale_exp(mx);
-  if (lane == 0) a_exp[m] = e;
+  const int e = min(scale_exp(mx), kExpMost);
+  if (lane == 0) a_exp[m] = static_cast<int8_t>(e - kExpBias);
 #pragma unroll
   for (int i = 0; i < kU; ++i) {
     const int k = (lane + i * kWave) * 4;
-    if (k >= kp) continue;
+    if (k >= K) continue;
     uint32_t h[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       h[j] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(tf32_rne_bits(v[i][j])), e)));
-    *reinterpret_cast<u32x2 *>(a + m * kp + k) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    *reinterpret_cast<u32x2 *>(a + m * K + k) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
   }
 }
 
@@ -246,15 +267,14 @@ bool router_dgrad_applies(int64_t K) { return K > 0 && K <= 320; }
 
 RouterDgradLayout router_dgrad_layout(int64_t M, int64_t K, int64_t N) {
   RouterDgradLayout l;
-  const int64_t kp = round64(K), M64 = round64(M);
   auto take = [&](int64_t bytes) {
     const size_t at = l.total;
     l.total += static_cast<size_t>(ceil_div(bytes, 256) * 256);
     return at;
   };
-  l.a = take(M64 * kp * 2);
-  l.b = take(N * kp * 2);
-  l.a_exp = take(M64 * 4);
+  l.a = take(M * K * 2);
+  l.b = take(K * N * 2);
+  l.a_exp = take(ceil_div(M, 4) * 4);
   l.b_exp = take(N * 4);
   return l;
 }
@@ -262,9 +282,10 @@ RouterDgradLayout router_dgrad_layout(int64_t M, int64_t K, int64_t N) {
 void launch_router_dgrad(const float *go, int64_t M, int64_t K, const float *w, int64_t N, float *out, void *workspace, hipStream_t s) {
   const RouterDgradLayout l = router_dgrad_layout(M, K, N);
   char *ws = static_cast<char *>(workspace);
-  const int64_t kp = round64(K), M64 = round64(M), wb = ceil_div(N, 64);
+  const int64_t wb = ceil_div(N, 64);
   uint16_t *a = reinterpret_cast<uint16_t *>(ws + l.a), *b = reinterpret_cast<uint16_t *>(ws + l.b);
-  int32_t *a_exp = reinterpret_cast<int32_t *>(ws + l.a_exp), *b_exp = reinterpret_cast<int32_t *>(ws + l.b_exp);
+  int8_t *a_exp = reinterpret_cast<int8_t *>(ws + l.a_exp);
+  int32_t *b_exp = reinterpret_cast<int32_t *>(ws + l.b_exp);
   DgradArgs p;
   p.a = a;
   p.b = b;
@@ -273,18 +294,19 @@ void launch_router_dgrad(const float *go, int64_t M, int64_t K, const float *w, 
   p.out = out;
   p.M = M;
   p.N = N;
+  p.K = static_cast<int>(K);
   p.col_tiles = static_cast<int>(ceil_div(N, kColsTile));
   // A unit for every CU, of whole stages.
   p.chunk = round64(std::max<int64_t>(64, ceil_div(M, std::max<int64_t>(1, num_cus() / p.col_tiles))));
   p.units = static_cast<int>(ceil_div(M, p.chunk)) * p.col_tiles;
-  const dim3 grid(static_cast<uint32_t>((p.units + 7) / 8 * 8)), block(512), pgrid(static_cast<uint32_t>(wb + M64 / 4));
+  const dim3 grid(static_cast<uint32_t>((p.units + 7) / 8 * 8)), block(512), pgrid(static_cast<uint32_t>(wb + ceil_div(M, 4)));
   auto go_ = [&](auto steps) {
     constexpr int kSteps = decltype(steps)::value;
-    router_dgrad_prepare_kernel<4 * kSteps><<<pgrid, dim3(256), 0, s>>>(w, go, M, M64, static_cast<int>(K), N, static_cast<int>(kp),
-                                                                        static_cast<int>(wb), a, b, a_exp, b_exp);
+    router_dgrad_prepare_kernel<4 * kSteps><<<pgrid, dim3(256), 0, s>>>(w, go, M, static_cast<int>(K), N, static_cast<int>(wb), a, b, a_exp,
+                                                                        b_exp);
     router_dgrad_kernel<kSteps><<<grid, block, 0, s>>>(p);
   };
-  switch (kp / 64) {
+  switch (ceil_div(K, 64)) {
     case 1: go_(std::integral_constant<int, 1>{}); break;
     case 2: go_(std::integral_constant<int, 2>{}); break;
     case 3: go_(std::integral_constant<int, 3>{}); break;

@@ -427,9 +427,8 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  * Limits: the column counts (K and N) % 8 == 0; dgrad 3K, N < 2^22 and
  *   3K*N < 2^30; wgrad M*N, M*K, N*K < 2^30; 16-byte aligned tensors.
  * Workspace: the *_workspace_size bytes, 256-byte aligned (dgrad: the fp16
- *   copies, M K + K N values (rounded up to 64 rows and, for K <= 320, 64
- *   reduction values), the row and column exponents and, for longer
- *   reductions, the column-max slabs; wgrad: the transposed fp16 copy of grad_output, its
+ *   copies, M K + K N values, the row and column exponents and, for K > 320,
+ *   the column-max slabs; wgrad: the transposed fp16 copy of grad_output, its
  *   columns' exponents and column-max slabs, and the fp32 planes of the
  *   reduction chunks with their columns' exponents where there are several; at least the size of an fp16
  *   copy of both operands with their exponents, slabs and planes). */

@@ -216,6 +216,19 @@ def test_workspace_sizes():
     assert lib.moe_router_wgrad_tf32_workspace_size(0, 16, 24) > 0  # one plane: the output is written through it
 
 
+@pytest.mark.parametrize("K", [8, 40, 64, 72, 128, 200, 256, 264, 320, 328])
+def test_router_dgrad_workspace_holds_the_copies_and_exponents(K):
+    # What callers that sized a workspace by the layout of the 128-row kernel hold is enough at every reduction length:
+    # fp16 copies of both operands, a byte per row (whole blocks of 128) and column, 4 bytes per column, the slabs.
+    def up(b):
+        return (b + 255) // 256 * 256
+    for M in (1, 5, 63, 64, 100, 1000, 16384, 100001):
+        for N in (8, 64, 520, 7168):
+            slabs = min(64, -(-K // 64))
+            most = up(2 * M * K) + up(2 * K * N) + up(-(-M // 128) * 128) + up(4 * N) + up(N) + up(4 * slabs * N)
+            assert 2 * M * K + 2 * K * N < L.lib().moe_router_dgrad_tf32_workspace_size(M, K, N) <= most, (M, N)
+
+
 def test_status_strings():
     lib = L.lib()
     for code in range(7):

@@ -276,3 +276,26 @@ def test_router_wgrad_tf32_sums_of_chunks_beyond_fp32(pkg, dev):
     got = pkg.ops.router_wgrad_tf32(go.to(dev), x.to(dev)).cpu().double()
     ref = go.double().t() @ x.double()  # all values are tf32 values
     assert torch.equal(got, ref), (got[0, :5], ref[0, :5])
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 8, 264), (65, 40, 520), (130, 200, 1032), (67, 264, 72)])
+def test_router_dgrad_tf32_partial_reduction_steps_and_tiny_rows(pkg, dev, M, K, N):
+    # Reductions that are not whole 64-value steps: what lies past a row's values is the next row's, here Inf and NaN, and
+    # must not reach the sums. Rows of subnormals only, down to the smallest that the rounding to tf32 leaves, take the
+    # largest exponent of their byte and stay exact (a sum of M exact products in fp32; results below 2^-126 round once
+    # more).
+    g = torch.Generator().manual_seed(M + K + N)
+    go = torch.randn(M, K, generator=g)
+    w = torch.randn(K, N, generator=g) * 2.0 ** 20
+    go[M // 2] = float("inf")
+    go[M // 2, 1::2] = float("nan")
+    go[0] = 2.0 ** -136
+    go[M - 1] *= 2.0 ** -127
+    w[:, N - 2] = float("nan")
+    got = pkg.ops.router_dgrad_tf32(go.to(dev), w.to(dev)).cpu().double()
+    rows = [m for m in range(M) if m != M // 2]
+    cols = [n for n in range(N) if n != N - 2]
+    assert bool(torch.isnan(got[M // 2]).all()) and bool(torch.isnan(got[:, N - 2]).all())
+    a, b = ref_torch.round_tf32_rne(go[rows]).double(), ref_torch.round_tf32_rne(w[:, cols]).double()
+    excess = (got[rows][:, cols] - a @ b).abs() - (K * 2.0 ** -24 * (a.abs() @ b.abs()) + 2.0 ** -149)
+    assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
