@@ -2450,41 +2450,50 @@ namespace {
 
 // Workspace of the tf32 wgrad (byte offsets, each 256-byte aligned): the transposed fp16 copy of grad_output, its
 // scale exponents, its column-max slabs, and the fp32 planes of the reduction chunks with the exponents of their columns
-// (none for one chunk). Its size is
-// never below `agreed`, what callers that sized their workspaces once were told: fp16 copies of both operands, both
-// operands' exponents and column-max slabs, and the planes of chunks of 512 rows or more.
+// (none for one chunk), as many as `bytes` hold.
 struct WgradTf32Layout {
   moe::RouterWgradPlan pl;
   moe::ColmaxPlan ca;
   size_t rows, exp, part, col_exp, planes, total;
 };
-WgradTf32Layout wgrad_tf32_layout(int64_t M, int64_t N, int64_t K) {
+WgradTf32Layout wgrad_tf32_layout(int64_t M, int64_t N, int64_t K, size_t bytes) {
   using moe::align_up;
   WgradTf32Layout l;
-  l.pl = moe::router_wgrad_plan(M, N, K);
   l.ca = moe::colmax_plan(M, N);
   size_t off = 0;
-  auto take = [&](size_t bytes) {
+  auto take = [&](size_t n) {
     const size_t at = off;
-    off += align_up(bytes);
+    off += align_up(n);
     return at;
   };
-  l.rows = take(static_cast<size_t>(moe::ceil_div(M, 64) * 64) * N * 2);
+  l.rows = take(static_cast<size_t>(moe::ceil_div(M, 8) * 8) * N * 2);
   l.exp = take(static_cast<size_t>(N) * 4);
   l.part = take(static_cast<size_t>(l.ca.S) * N * 4);
+  const size_t left = bytes > off ? std::min(bytes - off, static_cast<size_t>(INT64_MAX)) : 0;
+  const size_t each = static_cast<size_t>(K) * 4 * (static_cast<size_t>(N) + 1);
+  size_t most = each > 0 ? left / each : 1;
+  while (most > 1 && align_up(most * K * 4) + align_up(most * N * K * 4) > left) --most;
+  l.pl = moe::router_wgrad_plan(M, N, K, static_cast<int64_t>(std::max<size_t>(most, 1)));
   l.col_exp = take(l.pl.s > 1 ? static_cast<size_t>(l.pl.s) * K * 4 : 0);
   l.planes = take(l.pl.s > 1 ? static_cast<size_t>(l.pl.s) * N * K * 4 : 0);
+  l.total = off;
+  return l;
+}
+// What a call needs, and callers that sized their workspaces once were told: fp16 copies of both operands, both operands'
+// exponents and column-max slabs, and the planes of chunks of 512 rows or more. It always holds the layout of one chunk
+// (grad_output's copy has at most 7 rows more, 14 N bytes; one plane alone has 4 N K), and more chunks where it has room
+// for them: at 16384 x 320 x 8192 all 8 (321 MB, of which 94 are used), at 1024 x 320 x 1024 3 of 8.
+size_t wgrad_tf32_need(int64_t M, int64_t N, int64_t K) {
+  using moe::align_up;
   const int64_t tiles = moe::ceil_div(N, 256) * moe::ceil_div(K, 256);
   int64_t chunks = 1;
   if (M > 0 && tiles > 0 && tiles < 256) {
     chunks = std::min<int64_t>({moe::ceil_div(256, tiles), std::max<int64_t>(1, M / 512), 64});
     if (chunks > 1) chunks = moe::ceil_div(M, moe::ceil_div(moe::ceil_div(M, chunks), 64) * 64);
   }
-  const size_t agreed = align_up(static_cast<size_t>(M) * N * 2) + align_up(static_cast<size_t>(M) * K * 2) + align_up(static_cast<size_t>(N) * 4) +
-                        align_up(static_cast<size_t>(K) * 4) + align_up(static_cast<size_t>(l.ca.S) * N * 4) +
-                        align_up(static_cast<size_t>(moe::colmax_plan(M, K).S) * K * 4) + align_up(static_cast<size_t>(chunks) * N * K * 4);
-  l.total = std::max(off, agreed);
-  return l;
+  return align_up(static_cast<size_t>(M) * N * 2) + align_up(static_cast<size_t>(M) * K * 2) + align_up(static_cast<size_t>(N) * 4) +
+         align_up(static_cast<size_t>(K) * 4) + align_up(static_cast<size_t>(moe::colmax_plan(M, N).S) * N * 4) +
+         align_up(static_cast<size_t>(moe::colmax_plan(M, K).S) * K * 4) + align_up(static_cast<size_t>(chunks) * N * K * 4);
 }
 
 }  // namespace
@@ -2493,7 +2502,7 @@ extern "C" {
 
 size_t moe_router_wgrad_tf32_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M < 0 || N < 0 || K < 0) return 0;
-  return wgrad_tf32_layout(M, N, K).total;
+  return std::max(wgrad_tf32_need(M, N, K), wgrad_tf32_layout(M, N, K, SIZE_MAX).total);
 }
 
 int moe_router_wgrad_tf32(const float *grad_output, int64_t M, int64_t N, const float *inp, int64_t K,
@@ -2515,11 +2524,12 @@ int moe_router_wgrad_tf32(const float *grad_output, int64_t M, int64_t N, const 
   if (!is_aligned(grad_output, 16) || !is_aligned(inp, 16) || !is_aligned(grad_weight, 16)) {
     return fail(MOE_ERR_ALIGN, "%s: grad_output, inp and grad_weight must be 16-byte aligned", fn);
   }
-  const WgradTf32Layout l = wgrad_tf32_layout(M, N, K);
-  if (workspace == nullptr || workspace_bytes < l.total || !is_aligned(workspace, kWsAlign)) {
-    return fail(MOE_ERR_WORKSPACE, "%s: a 256-byte aligned workspace of %zu bytes is needed (got %zu)", fn, l.total,
+  const size_t need = wgrad_tf32_need(M, N, K);
+  if (workspace == nullptr || workspace_bytes < need || !is_aligned(workspace, kWsAlign)) {
+    return fail(MOE_ERR_WORKSPACE, "%s: a 256-byte aligned workspace of %zu bytes is needed (got %zu)", fn, need,
                 workspace == nullptr ? size_t(0) : workspace_bytes);
   }
+  const WgradTf32Layout l = wgrad_tf32_layout(M, N, K, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *w = static_cast<char *>(workspace);
   uint16_t *rows = reinterpret_cast<uint16_t *>(w + l.rows);

@@ -40,23 +40,25 @@ typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
 constexpr int kColsWave = 32, kColsTile = 256;
 constexpr int kRowB = kBK * 2;  // 128 bytes: one row of the small operand in a stage
 constexpr int64_t kWideK = int64_t(1) << 22;
+constexpr uint32_t kSkip = 0xfffffff0u;  // an offset past rows, which may span a little more than 2 GiB
 constexpr float kF16Max = 65504.f;
 constexpr int kNoExp = 1 << 20;  // a column without a finite nonzero value yet: its sums are 0, Inf or NaN, whatever the scale
 
 __device__ __forceinline__ int swz128(int row) { return (row >> 1) & 7; }
 
 struct WgradArgs {
-  const uint16_t *rows;  // [N, M64] fp16
+  const uint16_t *rows;  // [N, M8] fp16
   const int32_t *exp;    // [N]
   const float *inp;      // [M, K]
   float *out;            // planes [s, N, K], or (one chunk) the result
   int32_t *col_exp;      // the planes' column exponents [s, K]
-  int64_t M, M64, N, K;
+  int64_t M, M8, N, K;   // M8: M rounded up to 8
   int64_t chunk;         // reduction rows of a chunk
   int col_tiles, row_tiles, units;
 };
 
-// kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets). kNt: non-temporal loads of it.
+// kWide: 64-bit addresses for inp (rows so long that 64 of them do not fit 32-bit offsets, or no room for the planes of
+// the chunks that 32-bit ones need). kNt: non-temporal loads of it.
 // kOne: one chunk, whose sums are scaled back here.
 template <int kMI, bool kWide, bool kNt, bool kOne>
 __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
@@ -82,22 +84,28 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
   [[maybe_unused]] const int halves = 2 * steps;
 
   // ---- the small operand: this wavefront's blocks wave + 8 j of 8 rows
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.rows + static_cast<int64_t>(n0) * p.M64 + m0,
-                                              static_cast<uint32_t>(((min<int64_t>(p.N - n0, kMI * 16) - 1) * p.M64 + p.M64 - m0) * 2));
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.rows + static_cast<int64_t>(n0) * p.M8 + m0,
+                                              static_cast<uint32_t>(((min<int64_t>(p.N - n0, kMI * 16) - 1) * p.M8 + p.M8 - m0) * 2));
   int a_off[kDma];
 #pragma unroll
   for (int j = 0; j < kDma; ++j) {
     const int r = (wave + 8 * j) * 8 + (lane >> 3);
-    a_off[j] = n0 + r < p.N ? static_cast<int>(static_cast<uint32_t>(r) * static_cast<uint32_t>(p.M64 * 2) +
+    a_off[j] = n0 + r < p.N ? static_cast<int>(static_cast<uint32_t>(r) * static_cast<uint32_t>(p.M8 * 2) +
                                                static_cast<uint32_t>(((lane & 7) ^ swz128(r)) << 4))
-                            : static_cast<int>(kNoAccess);
+                            : static_cast<int>(kSkip);
   }
-  // Stage st into its slot; past the last one the last one again, into a slot that nothing reads any more.
+  // Stage st into its slot; past the last one the last one again, into a slot that nothing reads any more. A lane's eight
+  // values are the same ones of every row (the swizzle depends on wave % 2 alone); past M8 they are the next row's, and
+  // none are read.
+  const int a_row = ((lane & 7) ^ swz128(wave * 8 + (lane >> 3))) * 8;
+  const int rows8 = static_cast<int>(p.M8 - m0 < p.chunk ? p.M8 - m0 : p.chunk);
   auto dma = [&](int st) {
     const uint32_t dst = lds + (st % kSlots) * kStage;
-    const int k = min(st, steps - 1) * kRowB;
+    const int sc = min(st, steps - 1), k = sc * kRowB;
+    const bool in = sc * kBK + a_row < rows8;
 #pragma unroll
-    for (int j = 0; j < kDma; ++j) dma16b(ra, (lds_void *)(uintptr_t)(dst + (wave + 8 * j) * 1024), a_off[j], k);
+    for (int j = 0; j < kDma; ++j)
+      dma16b(ra, (lds_void *)(uintptr_t)(dst + (wave + 8 * j) * 1024), in ? a_off[j] : static_cast<int>(kSkip), k);
   };
 
   // ---- inp: columns col, col + 1, rows 32 h + 8 q + r of half h; rows past the chunk and columns past K read zeros
@@ -249,7 +257,7 @@ __global__ __launch_bounds__(512) void router_wgrad_kernel(WgradArgs p) {
 
 // Block (x, y): reduction rows 64 x .. + 63 and columns 64 y .. + 63 of grad_output, transposed through LDS. Each block
 // forms its columns' exponents from the slab maxima; those of x = 0 write them.
-__global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src, int64_t M, int64_t M64, int64_t N, const float *part,
+__global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src, int64_t M, int64_t M8, int64_t N, const float *part,
                                                                 int slabs, uint16_t *dst, int32_t *exp) {
   __shared__ int ex[64];
   __shared__ float red[4][64];
@@ -270,7 +278,7 @@ __global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src
     if (blockIdx.x == 0 && n0 + t < N) exp[n0 + t] = e;
   }
   __syncthreads();
-  if (m0 >= M64) return;  // M = 0: the exponents only
+  if (m0 >= M8) return;  // M = 0: the exponents only
   {
     const int c = (t & 15) * 4;  // N % 8 == 0: the four columns are all valid or all past N
 #pragma unroll
@@ -288,11 +296,11 @@ __global__ __launch_bounds__(256) void router_wgrad_rows_kernel(const float *src
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int c = (t >> 3) + 32 * k, r = (t & 7) * 8;
-    if (n0 + c >= N) continue;
+    if (n0 + c >= N || m0 + r >= M8) continue;
     uint32_t w[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const uint32_t *>(&tile[c][r + 2 * i]);
-    *reinterpret_cast<u32x4 *>(dst + (n0 + c) * M64 + m0 + r) = u32x4{w[0], w[1], w[2], w[3]};
+    *reinterpret_cast<u32x4 *>(dst + (n0 + c) * M8 + m0 + r) = u32x4{w[0], w[1], w[2], w[3]};
   }
 }
 
@@ -325,17 +333,25 @@ __global__ __launch_bounds__(256) void router_wgrad_sum_kernel(const float *plan
 
 }  // namespace
 
-RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K) {
+RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K, int64_t most_chunks) {
   RouterWgradPlan pl;
   pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 320));
   const int64_t blocks = ceil_div(ceil_div(std::max<int64_t>(N, 1), pl.row_tiles), 16);
-  pl.mi = K >= kWideK || blocks <= 4 ? 4 : blocks <= 8 ? 8 : blocks <= 16 ? 16 : 20;
+  pl.wide = K >= kWideK;
+  pl.mi = pl.wide || blocks <= 4 ? 4 : blocks <= 8 ? 8 : blocks <= 16 ? 16 : 20;
   pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 16 * pl.mi));
   const int64_t tiles = pl.row_tiles * std::max<int64_t>(1, ceil_div(K, kColsTile));
   // At most a unit for every CU (a second round for a few more costs a whole one: 16384 x 64 x 7168, 28 tiles, 10 chunks
   // 139 us, 9 101), of at least 128 rows; and a chunk of inp below 2 GiB (32-bit offsets).
-  int64_t s = std::max<int64_t>(1, std::min(256 / tiles, M / 128));
-  if (K < kWideK) s = std::max(s, ceil_div(M * K, (int64_t(1) << 29) - 64 * K));
+  const int64_t least = pl.wide ? 1 : std::max<int64_t>(1, ceil_div(M * K, (int64_t(1) << 29) - 64 * K));
+  int64_t s = std::max(least, std::min(256 / tiles, M / 128));
+  s = std::min(s, most_chunks);
+  if (s < least) {
+    s = 1;
+    pl.wide = true;
+    pl.mi = 4;
+    pl.row_tiles = std::max<int64_t>(1, ceil_div(N, 64));
+  }
   pl.c = std::max<int64_t>(1, ceil_div(ceil_div(M, s), kBK)) * kBK;
   pl.s = std::max<int64_t>(1, ceil_div(M, pl.c));
   return pl;
@@ -343,9 +359,8 @@ RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K) {
 
 void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, const float *part, int slabs, uint16_t *rows, int32_t *exp,
                               hipStream_t s) {
-  const int64_t M64 = ceil_div(M, 64) * 64;
-  router_wgrad_rows_kernel<<<dim3(static_cast<uint32_t>(std::max<int64_t>(1, M64 / 64)), static_cast<uint32_t>(ceil_div(N, 64))), dim3(256), 0,
-                             s>>>(grad_output, M, M64, N, part, slabs, rows, exp);
+  router_wgrad_rows_kernel<<<dim3(static_cast<uint32_t>(std::max<int64_t>(1, ceil_div(M, 64))), static_cast<uint32_t>(ceil_div(N, 64))),
+                             dim3(256), 0, s>>>(grad_output, M, ceil_div(M, 8) * 8, N, part, slabs, rows, exp);
 }
 
 void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const int32_t *exp, const float *inp, int64_t M, int64_t N,
@@ -357,7 +372,7 @@ void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const 
   p.out = pl.s > 1 ? planes : out;
   p.col_exp = col_exp;
   p.M = M;
-  p.M64 = ceil_div(M, 64) * 64;
+  p.M8 = ceil_div(M, 8) * 8;
   p.N = N;
   p.K = K;
   p.chunk = pl.c;
@@ -378,7 +393,7 @@ void launch_router_wgrad(const RouterWgradPlan &pl, const uint16_t *rows, const 
     }
   };
   const bool nt = M * K > 96 << 20;
-  if (K >= kWideK) router_wgrad_kernel<4, true, false, true><<<grid, block, 0, s>>>(p);  // (fewer than 256 rows: one chunk)
+  if (pl.wide) router_wgrad_kernel<4, true, false, true><<<grid, block, 0, s>>>(p);  // (one chunk)
   else if (pl.s == 1) go(std::false_type{}, std::true_type{});
   else if (nt) go(std::true_type{}, std::false_type{});
   else go(std::false_type{}, std::false_type{});

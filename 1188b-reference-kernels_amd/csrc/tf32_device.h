@@ -34,12 +34,14 @@ __device__ __forceinline__ int scale_exp(float mx) {
 // The work: ceil(K / 256) column tiles x row tiles of 16 mi rows x s reduction chunks of c rows (a multiple of 64).
 struct RouterWgradPlan {
   int mi;
+  bool wide;  // 64-bit addresses
   int64_t row_tiles, s, c;
 };
-RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K);
+// most_chunks (>= 1): for how many there is room.
+RouterWgradPlan router_wgrad_plan(int64_t M, int64_t N, int64_t K, int64_t most_chunks);
 
-// grad_output [M, N] fp32 -> its transpose in fp16, [N, M64] (M64 = M rounded up to 64, zeros past M), each row scaled
-// by 2^exp[n]; exp[n] from the column maxima of `slabs` slabs (part [slabs, N]).
+// grad_output [M, N] fp32 -> its transpose in fp16, [N, M8] (M8 = M rounded up to 8, zeros past M), each row scaled by
+// 2^exp[n]; exp[n] from the column maxima of `slabs` slabs (part [slabs, N]).
 void launch_router_wgrad_rows(const float *grad_output, int64_t M, int64_t N, const float *part, int slabs, uint16_t *rows, int32_t *exp,
                               hipStream_t s);
 // planes[chunk][N][K], scaled by exp and col_exp[chunk][K], then their sum in chunk order, scaled back (s == 1: the result

@@ -430,8 +430,10 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  *   copies, M K + K N values, the row and column exponents and, for K > 320,
  *   the column-max slabs; wgrad: the transposed fp16 copy of grad_output, its
  *   columns' exponents and column-max slabs, and the fp32 planes of the
- *   reduction chunks with their columns' exponents where there are several; at least the size of an fp16
- *   copy of both operands with their exponents, slabs and planes). */
+ *   reduction chunks with their columns' exponents where there are several; at
+ *   least an fp16 copy of both operands with their exponents, slabs and the
+ *   planes of chunks of 512 rows or more. A workspace of that least size is
+ *   enough; a larger one takes more chunks, in another order of the sums). */
 size_t moe_router_dgrad_tf32_workspace_size(int64_t M, int64_t K, int64_t N);
 int moe_router_dgrad_tf32(const float *grad_output, int64_t M, int64_t K, const float *weight, int64_t N,
                           float *grad_input, void *workspace, size_t workspace_bytes, void *stream);

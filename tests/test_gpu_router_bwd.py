@@ -299,3 +299,69 @@ def test_router_dgrad_tf32_partial_reduction_steps_and_tiny_rows(pkg, dev, M, K,
     a, b = ref_torch.round_tf32_rne(go[rows]).double(), ref_torch.round_tf32_rne(w[:, cols]).double()
     excess = (got[rows][:, cols] - a @ b).abs() - (K * 2.0 ** -24 * (a.abs() @ b.abs()) + 2.0 ** -149)
     assert bool((excess <= 0).all()), f"worst excess {excess.max().item():.3e}"
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1024, 320, 1024),  # planes for 3 chunks instead of 8
+    (700, 320, 520),    # 2 instead of 5
+    (200, 72, 8),       # one chunk
+    (4096, 64, 1000),   # all of them
+    (1, 1024, 8), (65, 520, 8), (70, 72, 24),  # the copy of grad_output is the larger part of the workspace
+])
+def test_router_wgrad_tf32_workspace_of_the_least_size(pkg, dev, M, N, K):
+    # fp16 copies of both operands, their exponents and column-max slabs and the planes of chunks of 512 rows or more are
+    # enough at every size, and nothing is stored past them. Inf and NaN in some columns of grad_output: the next row of
+    # its transposed copy is not read as the end of one.
+    def up(b):
+        return (b + 255) // 256 * 256
+    def slabs(rows):
+        s = max(1, min(64, -(-rows // 64)))
+        return -(-rows // -(-rows // s))
+    tiles = -(-N // 256) * -(-K // 256)
+    chunks = min(-(-256 // tiles), max(1, M // 512), 64)
+    if chunks > 1:
+        chunks = -(-M // (-(-(-(-M // chunks)) // 64) * 64))
+    least = (up(2 * M * N) + up(2 * M * K) + up(4 * N) + up(4 * K) + up(4 * slabs(M) * N) + up(4 * slabs(M) * K) + up(4 * chunks * N * K))
+    assert least <= pkg._lib.lib().moe_router_wgrad_tf32_workspace_size(M, N, K)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    go = torch.randn(M, N, generator=g, device=dev)
+    x = torch.randn(M, K, generator=g, device=dev)
+    go[0, 4] = float("inf")
+    go[M - 1, 6] = float("nan")
+    guard = 4096
+    ws = torch.full((least + guard,), 0xAB, dtype=torch.uint8, device=dev)
+    out = torch.empty(N, K, device=dev)
+    args = (pkg._lib.ptr(go), M, N, pkg._lib.ptr(x), K, pkg._lib.ptr(out), pkg._lib.ptr(ws))
+    with pytest.raises(pkg._lib.MoeError):
+        pkg._lib.call("moe_router_wgrad_tf32", *args, least - 1, pkg._lib.stream_handle())
+    pkg._lib.call("moe_router_wgrad_tf32", *args, least, pkg._lib.stream_handle())
+    assert bool((ws[least:] == 0xAB).all()), "stored past the workspace"
+    rows = [n for n in range(N) if n not in (4, 6)]
+    a, b = ref_torch.round_tf32_rne(go.cpu()[:, rows]).double(), ref_torch.round_tf32_rne(x.cpu()).double()
+    err = (out.cpu().double()[rows] - a.t() @ b).abs()
+    assert bool((err <= 1e-4 * (a.abs().t() @ b.abs()) + 1e-5).all()), f"worst error {err.max().item():.3e}"
+    assert not bool(torch.isfinite(out[4]).any()) and bool(torch.isnan(out[6]).all())
+
+
+def test_router_wgrad_tf32_chunks_that_do_not_fit_the_workspace(pkg, dev):
+    # inp of 2 GiB takes two chunks for its 32-bit offsets; a workspace without room for two planes of 2 GiB takes one,
+    # with 64-bit addresses. Some rows of the result against float64, at the bound of this file.
+    M, N, K = 8192, 8192, 65536
+    def up(b):
+        return (b + 255) // 256 * 256
+    least = up(2 * M * N) + up(2 * M * K) + up(4 * N) + up(4 * K) + up(4 * 64 * N) + up(4 * 64 * K) + up(4 * N * K)
+    assert least < pkg._lib.lib().moe_router_wgrad_tf32_workspace_size(M, N, K)
+    g = torch.Generator(device=dev).manual_seed(5)
+    go = torch.randn(M, N, generator=g, device=dev)
+    x = torch.randn(M, K, generator=g, device=dev)
+    ws = torch.empty(least, dtype=torch.uint8, device=dev)
+    out = torch.empty(N, K, device=dev)
+    pkg._lib.call("moe_router_wgrad_tf32", pkg._lib.ptr(go), M, N, pkg._lib.ptr(x), K, pkg._lib.ptr(out), pkg._lib.ptr(ws), least,
+                  pkg._lib.stream_handle())
+    del ws
+    rows = torch.tensor([0, 63, 64, 4097, N - 1], device=dev)
+    a = ref_torch.round_tf32_rne(go[:, rows]).double()
+    for at in range(0, K, 8192):
+        b = ref_torch.round_tf32_rne(x[:, at:at + 8192]).double()
+        err = (out[rows, at:at + 8192].double() - a.t() @ b).abs()
+        assert bool((err <= 1e-4 * (a.abs().t() @ b.abs()) + 1e-5).all()), f"columns from {at}: worst error {err.max().item():.3e}"
