@@ -139,41 +139,40 @@ __device__ __forceinline__ bool has_tail(int64_t m) {
 // 256-row tiles of a group of m rows when its tail (if has_tail) is left to the list.
 __device__ __forceinline__ int main_row_tiles(int m) { return (m + 255 - kTailMaxRows) / 256; }
 
-// The list, by one wavefront: each lane counts the tails of its chunk of
-// groups, an exclusive scan over the lanes gives the chunk's first list
-// position, then each lane lists its chunk's tail groups. Group g is rows
-// offsets[g] .. offsets[g + 1] - 1, clamped to [0, M]. If no group has more
-// than `shorts` rows, another kernel computes them all (kTailNone).
+// The list, by one wavefront: 64 neighbouring groups at a time, a lane each, ranked by a ballot; sixteen such sets are loaded
+// before the first of them is ranked. Group g is rows offsets[g] .. offsets[g + 1] - 1, clamped to [0, M]. If no group has
+// more than `shorts` rows, another kernel computes them all (kTailNone).
+// Measured (MI355X, us for the launch of 64, 1024 and 4096 groups): 4.8, 4.8 and 7.4; a run of groups for each lane, walked
+// twice: 4.8, 7.2 and 23.3, by 256 threads 4.8, 5.8 and 9.6.
 __device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails, int64_t shorts) {
-  const int lane = lane_id();
-  const int64_t per = (G + kWave - 1) / kWave;
-  const int64_t g0 = min(G, lane * per), g1 = min(G, g0 + per);
-  auto rows = [&](int64_t g) {
-    const int64_t lo = min(max(static_cast<int64_t>(offsets[g]), int64_t(0)), M);
-    return min(max(static_cast<int64_t>(offsets[g + 1]), lo), M) - lo;
-  };
-  int n = 0;
+  constexpr int kSets = 16;
+  const int lane = lane_id(), n = static_cast<int>(G), rows = static_cast<int>(M);  // M < 2^31
+  int pos = 0;
   bool longer = false;
-  for (int64_t g = g0; g < g1; ++g) {
-    const int64_t m = rows(g);
-    n += has_tail(m) ? 1 : 0;
-    longer |= m > shorts;
+  for (int g0 = 0; g0 < n; g0 += kSets * kWave) {
+    int lo[kSets], hi[kSets];
+#pragma unroll
+    for (int i = 0; i < kSets; ++i) {
+      const int g = min(g0 + i * kWave + lane, n - 1);
+      lo[i] = offsets[g];
+      hi[i] = offsets[g + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < kSets; ++i) {
+      const int g = g0 + i * kWave + lane;
+      const int first = min(max(lo[i], 0), rows);
+      const int m = g < n ? min(max(hi[i], first), rows) - first : 0;
+      const uint64_t tail = __ballot(has_tail(m));
+      if (has_tail(m)) tails[kTailList + pos + lanes_below(tail)] = g;
+      pos += __popcll(tail);
+      longer |= m > shorts;
+    }
   }
   const bool any_longer = __ballot(longer) != 0;
-  int pos = n;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int o = __shfl_up(pos, d);
-    pos += lane >= d ? o : 0;
-  }
-  if (lane == kWave - 1) {
+  if (lane == 0) {
     tails[kTailCount] = pos;
     tails[kTailNone] = any_longer ? 0 : 1;
     tails[kTailCtr] = 0;
-  }
-  pos -= n;
-  for (int64_t g = g0; g < g1; ++g) {
-    if (has_tail(rows(g))) tails[kTailList + pos++] = static_cast<int>(g);
   }
 }
 

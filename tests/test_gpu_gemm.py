@@ -290,3 +290,35 @@ def test_short_group_kernel_bit_identical(pkg, dev, sizes, K, N):
     assert torch.equal(again.view(torch.int16), pp.view(torch.int16))
     assert torch.isnan(buf[M * N:].float()).all()
     _sampled_check(x, w, offs.cpu(), out, False, rows_per_group=8)
+
+
+@pytest.mark.parametrize("G,cycle,gather", [
+    (2100, [0, 5, 130, 256, 300, 600, 128, 129], False),  # the list's own launch, more than two rounds of its loads
+    (1089, [0, 3, 200, 1, 60, 0, 20], True),              # made by the weight stream, which leaves the groups to it
+])
+def test_tail_list_of_many_groups(pkg, dev, G, cycle, gather):
+    """More groups than the list's kernel loads at a time: every tail is listed, once, at its own place. A missed or
+    doubled entry would leave rows of the output as they were; against 256-row tiles throughout, bit for bit."""
+    K, N = 192, 64
+    sizes = [cycle[i % len(cycle)] for i in range(G)]
+    M = sum(sizes)
+    g = torch.Generator(device=dev).manual_seed(G)
+    w = (torch.randn(G, N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    offs = pkg.ops.group_offsets_from_splits(sizes, dev)
+    nbytes = pkg.ops._lib.lib().moe_grouped_gemm_workspace_size(M, K, N, G)
+    assert nbytes >= 4 * (64 + G)
+    ws = torch.full((nbytes,), 0xAB, dtype=torch.uint8, device=dev)
+    none = torch.empty(0, dtype=torch.uint8, device=dev)
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=dev)
+    if gather:
+        rows = torch.arange(M, dtype=torch.int32, device=dev)
+        pkg.ops.grouped_gemm_gather(x, rows, w, offs, out=out, workspace=ws)
+        full = pkg.ops.grouped_gemm_gather(x, rows, w, offs, workspace=none)
+    else:
+        pkg.ops.grouped_gemm(x, w, offs, out=out, workspace=ws)
+        full = pkg.ops.grouped_gemm(x, w, offs, workspace=none)
+    assert torch.equal(out.view(torch.int16), full.view(torch.int16))
+    tails = [i for i, m in enumerate(sizes) if 1 <= m % 256 <= 128]
+    words = ws.view(torch.int32).cpu()
+    assert int(words[32]) == len(tails) and words[64:64 + len(tails)].tolist() == tails
