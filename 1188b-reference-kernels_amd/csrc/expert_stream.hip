@@ -402,7 +402,7 @@ __global__ __launch_bounds__(512) void expert_stream_kernel(GemmArgs p) {
   if (p.tails != nullptr) {
     // Only if every group is short; otherwise the ping-pong kernel that follows takes them all, and needs its list.
     if (tiles[0] > 0) {
-      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails, 0);
+      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails);
       return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) no_tails(p.tails);

@@ -140,15 +140,13 @@ __device__ __forceinline__ bool has_tail(int64_t m) {
 __device__ __forceinline__ int main_row_tiles(int m) { return (m + 255 - kTailMaxRows) / 256; }
 
 // The list, by one wavefront: 64 neighbouring groups at a time, a lane each, ranked by a ballot; sixteen such sets are loaded
-// before the first of them is ranked. Group g is rows offsets[g] .. offsets[g + 1] - 1, clamped to [0, M]. If no group has
-// more than `shorts` rows, another kernel computes them all (kTailNone).
+// before the first of them is ranked. Group g is rows offsets[g] .. offsets[g + 1] - 1, clamped to [0, M].
 // Measured (MI355X, us for the launch of 64, 1024 and 4096 groups): 4.8, 4.8 and 7.4; a run of groups for each lane, walked
 // twice: 4.8, 7.2 and 23.3, by 256 threads 4.8, 5.8 and 9.6.
-__device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails, int64_t shorts) {
+__device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
   constexpr int kSets = 16;
   const int lane = lane_id(), n = static_cast<int>(G), rows = static_cast<int>(M);  // M < 2^31
   int pos = 0;
-  bool longer = false;
   for (int g0 = 0; g0 < n; g0 += kSets * kWave) {
     int lo[kSets], hi[kSets];
 #pragma unroll
@@ -165,13 +163,11 @@ __device__ __forceinline__ void tails_list(const int32_t *offsets, int64_t G, in
       const uint64_t tail = __ballot(has_tail(m));
       if (has_tail(m)) tails[kTailList + pos + lanes_below(tail)] = g;
       pos += __popcll(tail);
-      longer |= m > shorts;
     }
   }
-  const bool any_longer = __ballot(longer) != 0;
   if (lane == 0) {
     tails[kTailCount] = pos;
-    tails[kTailNone] = any_longer ? 0 : 1;
+    tails[kTailNone] = 0;
     tails[kTailCtr] = 0;
   }
 }
@@ -185,9 +181,8 @@ __device__ __forceinline__ void no_tails(int *tails) {
 
 namespace {
 
-__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails,
-                                                       int64_t shorts) {
-  tails_list(offsets, G, M, tails, shorts);
+__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
+  tails_list(offsets, G, M, tails);
 }
 
 }  // namespace

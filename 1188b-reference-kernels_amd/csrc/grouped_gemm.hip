@@ -1520,8 +1520,26 @@ __global__ __launch_bounds__(512) void grouped_gemm_fwd128_kernel(GemmArgs p) {
   const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
   const int m32 = static_cast<int>(p.M), g_count = static_cast<int>(p.G);
   const int ntl = static_cast<int>((N + kTN - 1) / kTN);
-  // Only if every group fits one row tile, where a list was made first; otherwise the ping-pong kernel takes them all.
-  if (p.tails != nullptr && ld_inv(p.tails, kTailNone) == 0) return;
+  if (p.tails != nullptr) {
+    // A group of several row tiles reads its weights for each of them: where there are enough such tiles for the size of a
+    // group's weights, the ping-pong kernel that follows takes all groups, and needs its list.
+    int n = 0;  // row tiles, and groups with rows from bit 16 on (M <= 128 G, G <= 4096)
+#pragma unroll 4
+    for (int g = lane; g < g_count; g += kWave) {
+      const int lo = min(max(p.offsets[g], 0), m32);
+      const int m = min(max(p.offsets[g + 1], lo), m32) - lo;
+      n += (m + kTM - 1) / kTM + (m > 0 ? 1 << 16 : 0);
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) n += __shfl_xor(n, d);
+    const int tiles = __builtin_amdgcn_readfirstlane(n & 0xffff), groups = __builtin_amdgcn_readfirstlane(n >> 16);
+    const int64_t weights = N * K;
+    if (tiles > groups && (weights >= 1 << 24 || N <= 1024 || (weights >= 1 << 23 ? 8 * tiles >= 9 * groups : 4 * tiles > 5 * groups))) {
+      if (blockIdx.x == 0 && wave == 0) tails_list(p.offsets, p.G, p.M, p.tails);
+      return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) no_tails(p.tails);
+  }
 
   // ---- tile walker (every wavefront walks the same tiles): group by group, row tile-major
   struct Tile {
@@ -1842,20 +1860,26 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
                        is_aligned(workspace, 256);
   // Groups of at most 128 rows on average: the kernels for short groups, where the groups are short. With a workspace
   // they look at the groups first and leave a skewed split, in which a few groups hold most of the rows, to the
-  // ping-pong kernel, whose tail list the launch that looks makes (a few us for the launches that find nothing to do).
+  // ping-pong kernel, whose tail list they then make (1 to 2.5 us where it finds nothing to do).
   // Plain, 1023 tokens over 64 experts top-8 (K 2048, N 7168): 588 us in 128-row tiles throughout, 426 us this way;
-  // 40 even groups of 102 rows (K 8192, N 5120): 664 us in 128-row tiles, 735 in the ping-pong kernel's. SwiGLU and
-  // gather, 64 even groups of 48 and 64 rows (K 7168, N 4096): 633 and 636 us in the ping-pong kernel's tail tiles,
-  // 574 and 603 streamed; of 100 rows 649 against 691.
+  // 40 even groups of 102 rows (K 8192, N 5120): 664 us in 128-row tiles, 735 in the ping-pong kernel's. What decides is
+  // the row tiles for each group with rows, the sooner the larger a group's weights (128-row tiles and ping-pong kernel,
+  // us; 64 groups unless said): N 8192, K 2560 at 1.03 tiles 561, 531, N 4096, K 7168 726, 694; N 7168, K 2048 at 1.03
+  // 388, 407, at 1.125 422, 391; N 4096, K 2048 228, 253 and 244, 243, 128 groups at 1.125 488, 452; N 2048, K 2048 at
+  // 1.25 138, 143, 128 groups at 1.27 282, 247; 320 groups N 2048, K 1024 at 1.15 315, 329, at 1.28 336, 324, but N 1024,
+  // K 1024 (columns that the narrow tiles do not divide) at 1.03 202, 193.
+  // SwiGLU and gather, 64 even groups of 48 and 64 rows (K 7168, N 4096): 633 and 636 us in the ping-pong kernel's tail
+  // tiles, 574 and 603 streamed; of 100 rows 649 against 691.
   bool list_made = false;
   if (pingpong && M_total <= 128 * G) {
-    // (No group has more than 128 rows if there are no more in all; and below 512 MB of weights, some 90 us, the second
-    // launch costs what it can save.)
+    // (No group has more than 128 rows if there are no more in all. Below 512 MB of weights the 128-row tiles run
+    // throughout, some 10 us faster in calls of 15 to 45 us, where a group's weights, read again, come from the caches:
+    // 16 groups, N 1024, K 1024, 1.4 tiles for each 18, 31 us. From about 2^26 weights on a skewed split runs up to a
+    // quarter longer this way: 16 groups, N 4096, K 2048, 1.4 tiles 87, 73, 128 groups, N 1024, K 1024 103, 94.)
     const bool look = tail_ws && M_total > 128 && (!in_place || G * N * K >= int64_t(1) << 28);
     if (look) p.tails = static_cast<int *>(workspace);
     if (in_place) {
       // Plain epilogue, A rows in place: 128-row tiles with their own loading wavefronts.
-      if (look) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails, 128);
       switch (MOE_GEMM_FWD128_NB ? MOE_GEMM_FWD128_NB : fwd128_nb(M_total, N, G, P)) {
         case 4: grouped_gemm_fwd128_kernel<4><<<dim3(P), dim3(512), 0, s>>>(p); break;
         case 5: grouped_gemm_fwd128_kernel<5><<<dim3(P), dim3(512), 0, s>>>(p); break;
@@ -1906,7 +1930,7 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
   }
   if (tail_ws) {
     p.tails = static_cast<int *>(workspace);
-    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails, 0);
+    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails);
   }
   if (pingpong && p.tails != nullptr) {
     if (swiglu) {

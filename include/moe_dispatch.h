@@ -286,7 +286,7 @@ int moe_index_select(const moe_bf16_t *src, int64_t src_rows, int64_t row_elems,
  *   the tails is there and no group turns out longer than 64; with A rows in
  *   place and MOE_EPILOGUE_NONE, groups of at most 128 rows on average (e.g.
  *   case03/04) run 128-row tiles of 128-192 columns, and with the workspace
- *   only if no group is longer than 128. All under the same conditions and in
+ *   only if few groups are longer than 128. All under the same conditions and in
  *   the same summation order: the same result bit for bit. */
 size_t moe_grouped_gemm_workspace_size(int64_t M_total, int64_t K, int64_t N, int64_t G);
 int moe_grouped_gemm(const moe_bf16_t *a, int64_t M_total, int64_t K, const moe_bf16_t *w,

@@ -93,3 +93,28 @@ def test_choice_by_group_sizes_plain_large(pkg, dev, sizes):
     ws = torch.full((512,), 0xAB, dtype=torch.uint8, device=dev)
     for _ in range(2):
         _same(pkg.ops.grouped_gemm(x, w, offs, workspace=ws), drained, "with a workspace")
+
+
+@pytest.mark.parametrize("N,K,sizes,tiles", [
+    (8192, 2048, [100] * 16 + [0], True),             # 2^24 weights a group: a row tile each
+    (8192, 2048, [129] + [100] * 15 + [0], False),    # one row tile more
+    (4096, 2048, [257, 0] + [100] * 31, True),        # 2^23: 34 row tiles of 32 groups, less than an eighth more
+    (4096, 2048, [257, 0, 257] + [90] * 30, False),   # 36 of 32: an eighth
+    (2048, 2048, [640, 0] + [90] * 19 + [640, 0] + [90] * 11 + [40] * 32, True),     # below: 72 of 64
+    (2048, 2048, [1200, 1200] + [40] * 62, False),    # 82 of 64: more than a quarter
+])
+def test_choice_by_row_tiles_plain_large(pkg, dev, N, K, sizes, tiles):
+    # The 128-row tiles keep groups of several row tiles where these are few for the size of a group's weights. Word 33
+    # of the workspace says who computed the groups; the results are the same bit for bit.
+    M, G = sum(sizes), len(sizes)
+    assert 32 * G < M <= 128 * G and G * N * K >= 1 << 28
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(G, N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    offs = pkg.ops.group_offsets_from_splits(sizes, dev)
+    drained = pkg.ops.grouped_gemm(x, w, offs, workspace=torch.empty(0, dtype=torch.uint8, device=dev))
+    nbytes = pkg._lib.lib().moe_grouped_gemm_workspace_size(M, K, N, G)
+    ws = torch.full((nbytes,), 0xAB, dtype=torch.uint8, device=dev)
+    for _ in range(2):
+        _same(pkg.ops.grouped_gemm(x, w, offs, workspace=ws), drained, "with a workspace")
+    assert int(ws.view(torch.int32)[33]) == (1 if tiles else 0)
