@@ -5,7 +5,8 @@
 // is built around the stores:
 //   * the weight stays where it is used: a wavefront owns 64 columns and holds all their MFMA fragments (40 of 16 bytes
 //     a lane at K = 320) in registers for its whole run; only grad_output's rows stream by, through a ring of three LDS
-//     stages of 64 rows that the 8 wavefronts (512 columns) share, with one barrier a stage;
+//     stages of 64 rows that the 8 wavefronts (512 columns; 2 or 4 where there are few rows) share, with one barrier a
+//     stage;
 //   * block j of a wavefront's four is columns 4 c + j, c = 0 .. 15, so a lane's four accumulators of a row are four
 //     neighbouring columns: one 16-byte store, 256 contiguous bytes of a row over 16 lanes;
 //   * nothing waits for the stores: they are older than the loads that the next stages wait for only by whole stages.
@@ -32,7 +33,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
-constexpr int kRowsStage = 64, kColsWave = 64, kColsTile = 512;
+constexpr int kRowsStage = 64, kColsWave = 64;
 // Rows' exponents as bytes: scale_exp is -113 to 163, and a row whose largest magnitude is below 2^-128 (above 142) is as
 // exact with 142: its values, multiples of 2^-149, become multiples of 2^-7 below 2^14.
 constexpr int kExpBias = 15, kExpMost = 127 + kExpBias;
@@ -49,15 +50,16 @@ struct DgradArgs {
   int col_tiles, units;
 };
 
-// kKS2: 64-deep steps of the reduction.
-template <int kKS2>
-__global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
+// kKS2: 64-deep steps of the reduction. kWaves: wavefronts of a workgroup.
+template <int kKS2, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void router_dgrad_kernel(DgradArgs p) {
+  constexpr int kColsTile = kWaves * kColsWave;
   constexpr int kKS = 2 * kKS2;                  // MFMAs per block
   constexpr int kRowB = 128 * kKS2;              // bytes of a row in LDS
   constexpr int kStage = kRowsStage * kRowB;     // 8 kKS2 KiB
   constexpr int kExp = kRowsStage * 4;           // the rows' exponents
   constexpr int kSlots = 3;
-  constexpr int kDma = kKS2;                     // 1 KiB blocks per wavefront and stage
+  constexpr int kDma = 8 * kKS2 / kWaves;        // 1 KiB blocks per wavefront and stage
   constexpr int kStores = kRowsStage / 16 * 4;   // per lane and stage
   constexpr int kLds = kSlots * (kStage + kExp);
   static_assert(kLds <= 160 * 1024, "LDS");
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
   const int64_t m0 = static_cast<int64_t>(u / p.col_tiles) * p.chunk, m1 = min(p.M, m0 + p.chunk);
   const int stages = static_cast<int>((m1 - m0 + kRowsStage - 1) / kRowsStage);
 
-  // ---- rows: block wave + 8 j of a stage; 16-byte chunks of a row are XORed with the row within each 128 bytes, those past
+  // ---- rows: block wave + kWaves j of a stage; 16-byte chunks of a row are XORed with the row within each 128 bytes, those past
   // K and rows past M read zeros. The offsets are formed anew for each stage (from a lane index the compiler takes for
   // another): the registers are the weight's.
   const int row_bytes = p.K * 2;
@@ -93,10 +95,10 @@ __global__ __launch_bounds__(512) void router_dgrad_kernel(DgradArgs p) {
     asm volatile("" : "+v"(ln));
 #pragma unroll
     for (int j = 0; j < kDma; ++j) {
-      const int at = (wave + 8 * j) * 64 + ln;  // chunk of the stage, as it lies in LDS
+      const int at = (wave + kWaves * j) * 64 + ln;  // chunk of the stage, as it lies in LDS
       const int r = at / (8 * kKS2), c = at % (8 * kKS2);
       const int from = ((c & ~7) | ((c ^ r) & 7)) * 16;
-      dma16b(ra, (lds_void *)(uintptr_t)(lds + slot * kStage + (wave + 8 * j) * 1024),
+      dma16b(ra, (lds_void *)(uintptr_t)(lds + slot * kStage + (wave + kWaves * j) * 1024),
              from < row_bytes ? r * row_bytes + from : static_cast<int>(kNoAccess), 0);
     }
   };
@@ -295,16 +297,23 @@ void launch_router_dgrad(const float *go, int64_t M, int64_t K, const float *w, 
   p.M = M;
   p.N = N;
   p.K = static_cast<int>(K);
-  p.col_tiles = static_cast<int>(ceil_div(N, kColsTile));
+  // The fewer columns a workgroup owns, the less weight it waits for at its start: 2 or 4 wavefronts where all units of one
+  // stage then have a CU each (us, 2, 4 and 8 wavefronts, reductions of 320: 16 x 2048 16.8, 18.0, 23.1; 1024 x 1024 18.2,
+  // 19.3, 23.7; 2048 x 2048, twice the CUs with 2, 25.5, 23.1, 27.6; 8192 x 4096, four times with 4, 78.6, 50.7, 45.1).
+  auto fits = [&](int64_t n) { return ceil_div(N, n * kColsWave) * ceil_div(M, kRowsStage) <= num_cus(); };
+  const int waves = fits(2) ? 2 : fits(4) ? 4 : 8;
+  p.col_tiles = static_cast<int>(ceil_div(N, waves * kColsWave));
   // A unit for every CU, of whole stages.
   p.chunk = round64(std::max<int64_t>(64, ceil_div(M, std::max<int64_t>(1, num_cus() / p.col_tiles))));
   p.units = static_cast<int>(ceil_div(M, p.chunk)) * p.col_tiles;
-  const dim3 grid(static_cast<uint32_t>((p.units + 7) / 8 * 8)), block(512), pgrid(static_cast<uint32_t>(wb + ceil_div(M, 4)));
+  const dim3 grid(static_cast<uint32_t>((p.units + 7) / 8 * 8)), pgrid(static_cast<uint32_t>(wb + ceil_div(M, 4)));
   auto go_ = [&](auto steps) {
     constexpr int kSteps = decltype(steps)::value;
     router_dgrad_prepare_kernel<4 * kSteps><<<pgrid, dim3(256), 0, s>>>(w, go, M, static_cast<int>(K), N, static_cast<int>(wb), a, b, a_exp,
                                                                         b_exp);
-    router_dgrad_kernel<kSteps><<<grid, block, 0, s>>>(p);
+    if (waves == 2) router_dgrad_kernel<kSteps, 2><<<grid, dim3(128), 0, s>>>(p);
+    else if (waves == 4) router_dgrad_kernel<kSteps, 4><<<grid, dim3(256), 0, s>>>(p);
+    else router_dgrad_kernel<kSteps, 8><<<grid, dim3(512), 0, s>>>(p);
   };
   switch (ceil_div(K, 64)) {
     case 1: go_(std::integral_constant<int, 1>{}); break;

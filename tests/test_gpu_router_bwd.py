@@ -365,3 +365,12 @@ def test_router_wgrad_tf32_chunks_that_do_not_fit_the_workspace(pkg, dev):
         b = ref_torch.round_tf32_rne(x[:, at:at + 8192]).double()
         err = (out[rows, at:at + 8192].double() - a.t() @ b).abs()
         assert bool((err <= 1e-4 * (a.abs().t() @ b.abs()) + 1e-5).all()), f"columns from {at}: worst error {err.max().item():.3e}"
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (1000, 320, 1032), (1, 8, 136),      # two wavefronts a workgroup: 9 column tiles, and one column past a tile
+    (3000, 320, 1032), (1100, 72, 3848), # four
+    (12800, 264, 1032),                  # eight, units of several stages
+])
+def test_router_dgrad_tf32_workgroups_of_fewer_columns(pkg, dev, M, K, N):
+    test_router_dgrad_tf32_edges(pkg, dev, M, K, N)
