@@ -392,12 +392,12 @@ struct TopkArgs {
   float *probs;
 };
 
-template <int kEPL>
+template <int kEPL, bool kSorted = true>
 __global__ __launch_bounds__(256) void router_topk_kernel(TopkArgs p) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
   if (t >= p.M) return;
   const float *row = p.logits + t * p.N;
-  topk_row<kEPL>([&](int e) { return row[e]; }, t, p.N, p.k, p.values, p.indices, p.routing_map, p.probs);
+  topk_row<kEPL, kSorted>([&](int e) { return row[e]; }, t, p.N, p.k, p.values, p.indices, p.routing_map, p.probs);
 }
 
 int launch(const char *fn, const moe_bf16_t *inp, int64_t M, int64_t K, const moe_bf16_t *weight, int64_t N,
@@ -478,6 +478,12 @@ int launch(const char *fn, const moe_bf16_t *inp, int64_t M, int64_t K, const mo
   t.routing_map = routing_map;
   t.probs = probs;
   const int64_t tgrid = ceil_div(M, 4);
+  if (nb >= 6 && topk_searches(M, k)) {
+    if (nb == 6) router_topk_kernel<6, false><<<dim3(tgrid), dim3(256), 0, s>>>(t);
+    else if (nb == 7) router_topk_kernel<7, false><<<dim3(tgrid), dim3(256), 0, s>>>(t);
+    else router_topk_kernel<8, false><<<dim3(tgrid), dim3(256), 0, s>>>(t);
+    return check_launch(fn);
+  }
   switch (nb) {
     case 1: router_topk_kernel<1><<<dim3(tgrid), dim3(256), 0, s>>>(t); break;
     case 2: router_topk_kernel<2><<<dim3(tgrid), dim3(256), 0, s>>>(t); break;

@@ -10,29 +10,31 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
 
-template <int kEPL>
+template <int kEPL, bool kSorted>
 __global__ __launch_bounds__(kThreads) void topk_kernel(const float *logits, int64_t T, int E, int k,
                                                         float *values, int64_t *indices,
                                                         uint8_t *routing_map, float *probs) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + threadIdx.x / kWave;
   if (t >= T) return;
   const float *row = logits + t * E;
-  topk_row<kEPL>([&](int e) { return row[e]; }, t, E, k, values, indices, routing_map, probs);
+  topk_row<kEPL, kSorted>([&](int e) { return row[e]; }, t, E, k, values, indices, routing_map, probs);
 }
 
-// go(n) with the slots per lane that E experts need (n = 64-element pieces, 16 above 512 experts).
+// go(n, sorted) with the slots per lane that E experts need (n = 64-element pieces, 16 above 512 experts).
 template <typename Go>
-void by_slots(int E, Go go) {
+void by_slots(int E, bool searched, Go go) {
+  const std::true_type sorted{};
+  const std::false_type unsorted{};
   switch ((E + kWave - 1) / kWave) {
-    case 1: go(std::integral_constant<int, 1>{}); break;
-    case 2: go(std::integral_constant<int, 2>{}); break;
-    case 3: go(std::integral_constant<int, 3>{}); break;
-    case 4: go(std::integral_constant<int, 4>{}); break;
-    case 5: go(std::integral_constant<int, 5>{}); break;
-    case 6: go(std::integral_constant<int, 6>{}); break;
-    case 7: go(std::integral_constant<int, 7>{}); break;
-    case 8: go(std::integral_constant<int, 8>{}); break;
-    default: go(std::integral_constant<int, 16>{}); break;
+    case 1: go(std::integral_constant<int, 1>{}, sorted); break;
+    case 2: go(std::integral_constant<int, 2>{}, sorted); break;
+    case 3: go(std::integral_constant<int, 3>{}, sorted); break;
+    case 4: go(std::integral_constant<int, 4>{}, sorted); break;
+    case 5: go(std::integral_constant<int, 5>{}, sorted); break;
+    case 6: searched ? go(std::integral_constant<int, 6>{}, unsorted) : go(std::integral_constant<int, 6>{}, sorted); break;
+    case 7: searched ? go(std::integral_constant<int, 7>{}, unsorted) : go(std::integral_constant<int, 7>{}, sorted); break;
+    case 8: searched ? go(std::integral_constant<int, 8>{}, unsorted) : go(std::integral_constant<int, 8>{}, sorted); break;
+    default: go(std::integral_constant<int, 16>{}, unsorted); break;
   }
 }
 
@@ -56,10 +58,10 @@ int moe_topk(const float *logits, int64_t T, int64_t E, int64_t k, float *values
   if (grid > 0x7fffffff) return fail(MOE_ERR_CAPACITY, "moe_topk: T=%lld too large", (long long)T);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int e = static_cast<int>(E), kk = static_cast<int>(k);
-  auto go = [&](auto epl) {
-    topk_kernel<decltype(epl)::value><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
+  auto go = [&](auto epl, auto sorted) {
+    topk_kernel<decltype(epl)::value, decltype(sorted)::value><<<dim3(grid), dim3(kThreads), 0, s>>>(logits, T, e, kk, values, indices, routing_map, probs);
   };
-  by_slots(e, go);
+  by_slots(e, topk_searches(T, k), go);
   return check_launch("moe_topk");
 }
 

@@ -20,7 +20,8 @@
 // the index always found by a second DPP chain and the winner's list searched
 // again every round, and with this form: 320 experts 29.5 and 19.3 (8 slots a lane
 // before, 5 now), 160 21.6 and 14.4, 64 10.6 and 9.7. Above 8 slots the sort costs
-// more than the searches (1024 experts: 58 against 50), so the list stays unsorted.
+// more than the searches (1024 experts: 58 against 50), so the list stays unsorted; so it does above 5 for one or two
+// selected of many rows (topk_searches).
 #pragma once
 
 #include "moe_common.h"
@@ -75,14 +76,19 @@ __device__ __forceinline__ float wave_sum_f32(float x) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Whether lists of 6 to 8 elements are searched every round instead of sorted once: for one or two rounds where the rows
+// fill the chip. us, sorted and searched: 16384 rows of 512, k = 1 12.4 and 9.9, k = 2 13.1 and 10.9; 32768 of 448, k = 1
+// 21.4 and 18.0; 2048 of 512, k = 2 4.3 and 4.0; but 93 of 512, k = 2 3.8 and 4.0, k = 4 4.3 and 5.0; 16384 of 320, k = 4
+// 8.7 and 8.9.
+inline bool topk_searches(int64_t rows, int64_t k) { return k <= 2 && rows >= 1024; }
+
 // Top-k of row t (elements load(e), e < E) by the calling wavefront; writes
 // values/indices [T, k] and, when non-null, routing_map [T, E] and probs [T, E].
-template <int kEPL, typename Load>
+template <int kEPL, bool kSorted = (kEPL <= 8), typename Load>
 __device__ __forceinline__ void topk_row(Load load, int64_t t, int E, int k, float *values, int64_t *indices,
                                          uint8_t *routing_map, float *probs) {
   const int lane = lane_id();
   float val[kEPL];
-  constexpr bool kSorted = kEPL <= 8;
   uint32_t key[kEPL], slot[kEPL];  // key 0 = nothing left (every float's order key is above 0)
 #pragma unroll
   for (int s = 0; s < kEPL; ++s) {

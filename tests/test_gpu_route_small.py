@@ -75,3 +75,30 @@ def test_row_id_map_more_than_one_round(pkg, dev, T, E):
     assert torch.equal(got["expert_major_i32"].cpu().long(), row_em)
     assert torch.equal(got["expert_offsets"].cpu(), ref_torch.expert_offsets(rm))
     assert torch.equal(got["src_token"].cpu().long(), rm.t().nonzero()[:, 1])
+
+
+@pytest.mark.parametrize("E", [320, 321, 384, 385, 448, 449, 512])
+@pytest.mark.parametrize("levels", [2, 0])
+def test_topk_one_or_two_of_many_rows(pkg, dev, E, levels):
+    # From 1024 rows on, lists of 6 to 8 elements a lane are searched for k = 1 and 2 and sorted for more; ties and special
+    # values as above. The router's fused top-k takes the same forms on its own logits.
+    g = torch.Generator().manual_seed(E + levels)
+    T = 1025
+    x = torch.randint(0, levels, (T, E), generator=g).float() if levels else torch.randn(T, E, generator=g)
+    special = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), 3.4e38])
+    hit = torch.rand(T, E, generator=g) < 0.02
+    x[hit] = special[torch.randint(0, 6, (int(hit.sum()),), generator=g)]
+    inp = torch.randn(T, 64, generator=g).to(torch.bfloat16).to(dev)
+    weight = (torch.randint(0, 3, (E, 64), generator=g) - 1).to(torch.bfloat16).to(dev) if levels else torch.randn(E, 64, generator=g).to(torch.bfloat16).to(dev)
+    logits = pkg.ops.router_logits(inp, weight)
+    for k in (1, 2, 3):
+        for rows in (T, 1023):
+            values, indices, mask = pkg.ops.topk(x[:rows].to(dev), k, with_mask=True)
+            rv, ri = ref_torch.topk(x[:rows], k)
+            assert torch.equal(indices.cpu(), ri), f"E={E} k={k} rows={rows}"
+            assert_bits_equal(values, rv, f"E={E} k={k} rows={rows}")
+            assert torch.equal(mask.cpu(), torch.zeros(rows, E, dtype=torch.bool).scatter_(1, ri, True))
+        fused = pkg.ops.router_topk(inp, weight, k)
+        rv, ri = ref_torch.topk(logits.cpu(), k)
+        assert torch.equal(fused[1].cpu(), ri), f"fused E={E} k={k}"
+        assert_bits_equal(fused[0], rv, f"fused E={E} k={k}")
