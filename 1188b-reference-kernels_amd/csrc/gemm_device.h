@@ -117,7 +117,7 @@ inline int num_cus() {
 
 // Tail list of the ping-pong kernels (workspace layout, ints): a group whose
 // last 256-row tile would have 1 to 128 rows leaves that tile to the 128-row
-// form of the kernel. tails_init_kernel lists those groups in order; after
+// form of the kernel. tails_list lists those groups in order; after
 // their 256-row tiles the persistent workgroups take (group, column tile)
 // units u = 0, 1, ... of the list from the counter, unit u = list[u / ntiles],
 // column tile u % ntiles.
@@ -179,13 +179,8 @@ __device__ __forceinline__ void no_tails(int *tails) {
   tails[kTailCtr] = 0;
 }
 
-namespace {
-
-__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
-  tails_list(offsets, G, M, tails);
-}
-
-}  // namespace
+// The list in a launch of its own, before a ping-pong kernel (grouped_gemm.hip).
+void launch_tails_init(const int32_t *offsets, int64_t G, int64_t M, int *tails, hipStream_t s);
 
 }  // namespace gemm
 }  // namespace moe

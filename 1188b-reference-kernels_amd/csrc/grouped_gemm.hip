@@ -1716,7 +1716,16 @@ __global__ __launch_bounds__(512) void grouped_gemm_fwd128_kernel(GemmArgs p) {
   }
 }
 
+__global__ __launch_bounds__(64) void tails_init_kernel(const int32_t *offsets, int64_t G, int64_t M, int *tails) {
+  tails_list(offsets, G, M, tails);
+}
+
 }  // namespace
+
+void gemm::launch_tails_init(const int32_t *offsets, int64_t G, int64_t M, int *tails, hipStream_t s) {
+  tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(offsets, G, M, tails);
+}
+
 }  // namespace moe
 
 namespace {
@@ -1930,7 +1939,7 @@ int launch_grouped_gemm(const char *fn, const moe_bf16_t *a, int64_t a_src_rows,
   }
   if (tail_ws) {
     p.tails = static_cast<int *>(workspace);
-    if (!list_made) tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(p.offsets, p.G, p.M, p.tails);
+    if (!list_made) launch_tails_init(p.offsets, p.G, p.M, p.tails, s);
   }
   if (pingpong && p.tails != nullptr) {
     if (swiglu) {

@@ -2246,7 +2246,7 @@ int moe_grouped_gemm_dgrad(const moe_bf16_t *dy, int64_t M_total, int64_t N, con
     if (dgrad_pp_tails(M_total, N, G) && workspace != nullptr && workspace_bytes >= gemm::tails_bytes(G) &&
         is_aligned(workspace, kWsAlign)) {
       p.tails = static_cast<int *>(workspace);
-      gemm::tails_init_kernel<<<dim3(1), dim3(64), 0, s>>>(group_offsets, G, M_total, p.tails);
+      gemm::launch_tails_init(group_offsets, G, M_total, p.tails, s);
       launch_pp<false, false, true>(p, (ceil_div(M_total, 256) + G) * p.ntiles, s);
     } else {
       launch_pp<false>(p, (ceil_div(M_total, 256) + G) * p.ntiles, s);
