@@ -51,3 +51,27 @@ def test_gemm_kernels_do_not_spill():
     assert all(v.get("agpr") in (128, 256) for name, v in rows if "gemm" in name and "kernel" in name and "sum_planes" not in name
                and "split" not in name and "tails_init" not in name and "_pp_kernel" not in name
                and "_sweep_kernel" not in name and "_fwd128_kernel" not in name and (name, v) not in dg128)
+
+
+def test_streaming_kernels_do_not_spill():
+    """The kernels of the weight stream and of the tf32 router backward count their vector-memory operations too: a spill's
+    scratch loads and stores would be among them. Workgroups of 512 threads need two wavefronts per SIMD."""
+    import resource_usage as ru
+    hipcc = ru._hipcc()
+    with ThreadPoolExecutor(max_workers=3) as ex:
+        results = list(ex.map(lambda s: ru.usage(s, hipcc), ["expert_stream.hip", "router_dgrad.hip", "router_wgrad.hip"]))
+    stream, dgrad, wgrad = results
+    spilled = [(name, v) for rows in results for name, v in rows if v.get("scratch", 0) != 0]
+    assert not spilled, spilled
+    # epilogue x gather; 5 reduction lengths x 2, 4 and 8 wavefronts; 4 row blocks x (plain, non-temporal, one chunk) and
+    # the form of 64-bit addresses
+    full = [r for r in stream if "expert_stream_kernel" in r[0]]
+    assert len(full) == 4, full
+    gemms = [r for r in dgrad if "router_dgrad_kernel" in r[0]]
+    assert len(gemms) == 15, gemms
+    full += [r for r in gemms if "Li8EEE" in r[0]]
+    assert len(full) == 9, full
+    units = [r for r in wgrad if "router_wgrad_kernel" in r[0]]
+    assert len(units) == 13, units
+    full += units
+    assert all(v.get("occ") >= 2 and v.get("vgpr", 0) + v.get("agpr", 0) <= 256 for _, v in full), full
