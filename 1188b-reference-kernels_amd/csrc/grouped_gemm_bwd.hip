@@ -73,7 +73,7 @@ struct BwdArgs {
   const uint16_t *a;        // dy [M, N]
   const uint16_t *b;        // dgrad: w [G, N, K]; wgrad: x [M, K]
   const int32_t *offsets;   // [G + 1], or nullptr: group g is rows [g chunk, (g + 1) chunk) of M
-  void *out;                // dgrad: dx [M, K]; wgrad: dw [G, N, K] (bf16, or fp32 for kOut != 0)
+  void *out;                // dgrad: dx [M, K] (bf16, or fp32 for kOut != 0); wgrad: dw [G, N, K] (bf16)
   int64_t M, N, K, G;
   int64_t ntiles;           // column tiles, ceil(K / 256)
   int64_t chunk;            // rows per group when offsets is nullptr
@@ -614,6 +614,7 @@ template <bool kWgrad, int kOut, bool kSplit = false, bool kOrder = false>
 __global__ __launch_bounds__(256) void grouped_gemm_bwd_pipe_kernel(BwdArgs p) {
   static_assert(!kSplit || (!kWgrad && kOut == 1), "the split is a dgrad with fp32 planes");
   static_assert(!kOrder || kWgrad, "the group order is a wgrad schedule");
+  static_assert(!kWgrad || kOut == 0, "wgrad writes bf16 (the tf32 router wgrad has a kernel of its own)");
   constexpr int kBM = 256;
   constexpr int kWaves = 4;
   constexpr int kThreads = 256;
