@@ -12,8 +12,9 @@
 //   * nothing waits for the stores: they are older than the loads that the next stages wait for only by whole stages.
 // grad_output is scaled per row, weight per column (transposed, so that both are read along the reduction), in one launch
 // before; the epilogue undoes both.
-// Measured (MI355X, us for the call): 16384 x 320 x 8192 232 -> 138 (the GEMM 209 -> 107-117: 4.6-5.0 TB/s of output;
-// its operands' preparation 25 in four launches -> 18 in one), 16384 x 64 x 7168 164 -> 98, 100 x 64 x 7168 24 -> 17.
+// Measured (MI355X, us for the call in a graph): 16384 x 320 x 8192 217 -> 125-140 (the GEMM 209 -> 107-122: 4.4-5.0 TB/s
+// of output; its operands' preparation 25 in four launches -> 18 in one), 16384 x 64 x 7168 163 -> 95, 1024 x 320 x 1024
+// 21.5 -> 18.2, 100 x 64 x 7168 19.0 -> 9.5.
 // Before: 128 x 128 tiles of five reduction steps, 32 bytes of a row per store, still what longer reductions run
 // (grouped_gemm_dgrad128_kernel in grouped_gemm_bwd.hip).
 #include <algorithm>

@@ -17,9 +17,10 @@
 //   * M is cut into chunks so that there is a unit for every CU; the units of one XCD share a chunk, whose part of the
 //     small operand then stays in its L2. The planes of the chunks stay scaled, each column with its chunk's exponent;
 //     they are brought to the column's smallest exponent, added in order and scaled back once.
-// Measured (MI355X, 16384 x 320 x 8192, us): 395 -> 171 for the whole call; the GEMM 120-134 (4.0-4.5 TB/s of inp; 150 without the multiplications and conversions, so it is the loads), the
-// planes' sum 16, grad_output's maxima and copy 17. Before: column maxima of inp 90, its fp16 copy 180, a GEMM on the
-// copies 143, the sum 10. 16384 x 64 x 7168: 307 -> 101; 4096 x 128 x 7168: 98 -> 49; 100 x 64 x 7168: 39 -> 19.
+// Measured (MI355X, 16384 x 320 x 8192, us, calls in a graph): 370 -> 157-167 for the whole call; the GEMM 122-135
+// (4.0-4.4 TB/s of inp; 150 for the call without the multiplications and conversions, so it is the loads), the planes' sum
+// 17, grad_output's maxima and copy 21. Before: column maxima of inp 90, its fp16 copy 180, a GEMM on the copies 143, the
+// sum 10. 16384 x 64 x 7168: 308 -> 100; 4096 x 128 x 7168: 100 -> 46; 1024 x 320 x 1024: 44 -> 33; 100 x 64 x 7168: 34 -> 19.
 #include <algorithm>
 #include <type_traits>
 

@@ -415,7 +415,8 @@ int moe_cast_f32_to_bf16(const float *src, int64_t n, moe_bf16_t *dst, void *str
  *     subnormal);
  *     the scale comes from the largest finite magnitude (Inf and NaN entries
  *     stay Inf and NaN), a row or column with no finite nonzero value keeps
- *     scale 1 (dgrad: one whose largest is below 2^-112 takes 2^127).
+ *     scale 1 (dgrad with K > 320: one whose largest is below 2^-112 takes
+ *     2^127).
  *   dgrad: grad_input [M, N] = tf32(grad_output [M, K]) @ tf32(weight [K, N]):
  *     grad_output scaled per row, weight per column, the scales undone in the
  *     GEMM's epilogue.
