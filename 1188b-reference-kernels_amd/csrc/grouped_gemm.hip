@@ -1789,9 +1789,12 @@ int fwd128_nb(int64_t M_total, int64_t N, int64_t G, int64_t P) {
   return best;
 }
 
-// Whether those tiles fill their rounds to 2%, and are wider than the stream's 128 columns or take one round only.
-// Then the 128-row kernel is as fast as the stream or faster (us, it and the stream: 40 groups of 16 rows, K 8192, N
-// 5120: 535, 544; one round: 8 groups of 11 rows, K 1344, N 6096: 24, 26; 4 of 25, K 1024, N 8192: 14, 17).
+// Whether those tiles fill their rounds to 2%, and are wider than the stream's 128 columns or take one round only: there
+// neither kernel is the faster one throughout, and the calls keep the tiles that they had (68 pairs of 4 to 128 groups of 8
+// to 32 rows; us, tiles and stream). Short calls of few groups are faster in tiles: 4 groups of 16 rows, N 8192, K 1024 13.4,
+// 15.2, K 2560 28.5, 30.6; 8 of 25, N 6096, K 1344 25.5, 26.3. Many groups are within 4% of each other with even splits
+// (128 of 16, N 3072, K 4096 553, 558; 40 of 16, N 5120, K 8192 562, 556) and up to 13% slower in tiles with skewed ones.
+// Few groups with long reductions are slower in tiles: 8 of 25, N 5120, K 8192 139, 124; 16 of 25, N 3072, K 4096 86, 79.
 bool fwd128_even(int64_t M_total, int64_t N, int64_t G, int64_t P) {
   const int nb = fwd128_nb(M_total, N, G, P);
   const int64_t tn = 32 * nb, rounds = moe::ceil_div(G * moe::ceil_div(N, tn), P);
