@@ -367,8 +367,9 @@ __global__ __launch_bounds__(512) void expert_stream_kernel(GemmArgs p) {
     const int simd = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_s_getreg((1 << 11) | (4 << 6) | 4)) & 3;
     volatile int *sid = reinterpret_cast<volatile int *>(smem);
     int n[3] = {0, 0, 0};
+#pragma unroll 4
     for (int g = threadIdx.x; g < static_cast<int>(p.G); g += 512) {
-      const int m = g == role.lane ? first.m : group_rows(p, g).m;
+      const int m = group_rows(p, g).m;
       n[0] += class_tiles<128>(m);
       n[1] += class_tiles<64>(m);
       n[2] += class_tiles<32>(m);

@@ -1523,6 +1523,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_fwd128_kernel(GemmArgs p) {
   if (p.tails != nullptr) {
     // A group of several row tiles reads its weights for each of them: where there are enough such tiles for the size of a
     // group's weights, the ping-pong kernel that follows takes all groups, and needs its list.
+    // (Each wavefront counts for itself: counts shared through LDS took 1145 us for 4096 even groups of 100 rows, N 512,
+    // K 256, and 498 for 1024 of N 1024, K 512, against 1030 and 458.)
     int n = 0;  // row tiles, and groups with rows from bit 16 on (M <= 128 G, G <= 4096)
 #pragma unroll 4
     for (int g = lane; g < g_count; g += kWave) {
