@@ -374,3 +374,16 @@ def test_router_wgrad_tf32_chunks_that_do_not_fit_the_workspace(pkg, dev):
 ])
 def test_router_dgrad_tf32_workgroups_of_fewer_columns(pkg, dev, M, K, N):
     test_router_dgrad_tf32_edges(pkg, dev, M, K, N)
+
+
+def test_router_dgrad_tf32_rows_near_the_largest_value(pkg, dev):
+    # The smallest exponent that a row's byte holds: largest magnitudes in [2^127, 2^128). The bound of a sum of K exact
+    # products in fp32.
+    M, K, N = 70, 64, 136
+    g = torch.Generator().manual_seed(3)
+    go = torch.randn(M, K, generator=g) * 2.0 ** 120
+    go[:, 5] = 1.5 * 2.0 ** 127
+    w = torch.randn(K, N, generator=g) * 2.0 ** -30
+    got = pkg.ops.router_dgrad_tf32(go.to(dev), w.to(dev)).cpu().double()
+    a, b = ref_torch.round_tf32_rne(go).double(), ref_torch.round_tf32_rne(w).double()
+    assert bool(((got - a @ b).abs() <= K * 2.0 ** -24 * (a.abs() @ b.abs())).all())
